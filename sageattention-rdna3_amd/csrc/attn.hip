@@ -119,6 +119,7 @@ __device__ uint64_t g_stamps[kStampBlocks * 8 * kStampStride];
 namespace w8 {
 constexpr int kBM = 256;
 constexpr int kWaves = 8;
+constexpr int kGroups = 1;
 constexpr int kBlocksPerCu = 1;
 constexpr bool kSmallShape = false;
 #include "attn_body.inc"
@@ -127,6 +128,7 @@ constexpr bool kSmallShape = false;
 namespace w4 {
 constexpr int kBM = 128;
 constexpr int kWaves = 4;
+constexpr int kGroups = 1;
 constexpr int kBlocksPerCu = 2;
 constexpr bool kSmallShape = true;
 #include "attn_body.inc"
