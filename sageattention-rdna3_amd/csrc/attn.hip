@@ -1,9 +1,9 @@
 // Fused flash attention for gfx950 (CDNA4, wave64 MFMA): the INT8 quantized
 // path and the direct fp16/bf16 path, one kernel template.  The kernels and
-// their host code live in attn_body.inc, compiled here in two block shapes;
+// their host code live in attn_body.inc, compiled here in three block shapes;
 // this file holds the C entry points, which pick the shape per launch.  The
-// mapping below describes the 256-row shape (8 waves); the 128-row shape has
-// 4 waves and two blocks per CU.
+// mapping below describes the 256-row shape (8 waves); the 128-row shapes have
+// 4 waves and two blocks per CU, or 8 waves in two key groups.
 //
 // Math (csrc/attn_gfx11.cu of the reference):
 //   INT8   (:409-825)   s_ij = float(sum_d q8[i,d] * k8[j,d]) * (q_scale[i/32] * k_scale[j/16])
@@ -90,20 +90,30 @@ int device_cus() {
 
 }  // namespace
 
-// The kernels and their host code in two block shapes (attn_body.inc):
+// The kernels and their host code in three block shapes (attn_body.inc):
 //   * w8: 8 waves x 32 query rows = 256-row q-blocks, one block per CU;
 //   * w4: 4 waves x 32 query rows = 128-row q-blocks, two blocks per CU, whose
 //     waves do not share barriers, so one block's prologue, epilogue and
 //     barrier waits overlap the other's key loop; each block loads its own K/V
-//     tiles (twice the L2->LDS traffic of w8).
-// w4 runs the D = 64 non-causal launches (direct and INT8) and the causal
-// launches with few q-blocks (small_blocks), w8 all others.  Same-box timings
+//     tiles (twice the L2->LDS traffic of w8);
+//   * g2: 2 key groups x 4 waves x 32 query rows = 128-row q-blocks, one block
+//     per CU: the groups take every other key tile of the same rows and merge
+//     in LDS.  A launch with at most one 128-row q-block per CU has two waves
+//     per SIMD this way and half the key steps; in w4 the lone block's one wave
+//     per SIMD issues alone (a D = 64 direct step 1.9k cycles, against 3.0k for
+//     two tiles in g2).
+// The 128-row shapes run the D = 64 non-causal launches (direct and INT8) and
+// the causal launches with few q-blocks (small_blocks; all of those in g2, the
+// D = 64 ones as key_groups picks), w8 all others.  Same-box timings of w4
 // against w8 (identical outputs): D = 64 non-causal -7% to -27% (the direct
 // kernel at B1 H20 S1024: 21.3 -> 15.6 us; INT8 at B1 H10 S4096: 65.9 -> 56.2
 // us); causal launches of one or more full rounds +2% to +6% and D = 128
 // non-causal launches with key splits +3% to +4% (the doubled tile traffic),
-// so those stay on w8.  The D = 128 direct kernel's 98 KB of LDS fits once per
-// CU: its w4 launches (causal, few q-blocks) run one block per CU.
+// so those stay on w8.  g2 against w4, whole sageattn, same box: INT8 causal
+// B1 H8 S4096 D128 64.8 -> 61.3 us, H4 S8192 107 -> 98; direct causal B1 H16
+// S2048 D128 46.3 -> 37.9, H8 S1024 D128 23.8 -> 22.4, H16 S2048 D64 29.2 ->
+// 27.1, H8 S7000 D64 (INT8) 77.3 -> 69.8, H32 S2048 D64 39.7 -> 38.6; paired
+// causal D128 within 1%; direct non-causal B1 H20 S1024 D64 19.7 -> 16.6.
 // The stamps build (build.py --stamps, SAGE_STAMPS=1) adds per-wave cycle
 // stamps to the attention kernels (attn_body.inc, StampField) and the two
 // functions below that read them; the default build has neither.
@@ -133,6 +143,15 @@ constexpr int kBlocksPerCu = 2;
 constexpr bool kSmallShape = true;
 #include "attn_body.inc"
 }  // namespace w4
+
+namespace g2 {
+constexpr int kBM = 128;
+constexpr int kWaves = 4;
+constexpr int kGroups = 2;
+constexpr int kBlocksPerCu = 1;
+constexpr bool kSmallShape = true;
+#include "attn_body.inc"
+}  // namespace g2
 
 // A lone 128-row block on a CU takes this fraction of a 256-row block's time
 // per key tile step (MI355X, B1 H32 S2048 causal: the D = 128 direct kernel
@@ -169,6 +188,25 @@ bool small_blocks(int64_t head_dim, int is_causal, int64_t batch, int64_t q_head
            w8::causal_blocks_cost<64, w8::kQkBf16>(batch * q_heads, q_len, kv_len);
   return f * w4::causal_blocks_cost<128, w4::kQkBf16>(batch * q_heads, q_len, kv_len) <
          w8::causal_blocks_cost<128, w8::kQkBf16>(batch * q_heads, q_len, kv_len);
+}
+
+// Whether a launch of 128-row q-blocks runs in g2 instead of w4: every causal
+// one (their blocks are alone on a CU in either shape), and a non-causal one
+// whose items (q-blocks, or key pieces of split ones) fit one per CU and have
+// at least this many key tiles.  With more items than CUs w4 hosts two blocks
+// a CU, which share no barrier (B1 H10 S4096 D64, 512 items: w4 60 us, g2 65);
+// with fewer tiles the merge and the doubled prologue outweigh the halved
+// steps (kernel alone, w4 / g2: 4 tiles 8.0 / 8.8 us, 8 tiles 10.6 / 10.9, 12
+// tiles 12.8 / 13.2, 16 tiles 19.7 / 16.9, 36 tiles whole call 31.8 / 29.6).
+constexpr int64_t kMinGroupTiles = 16;
+bool key_groups(int is_causal, int64_t head_dim, int64_t batch, int64_t q_heads, int64_t q_len, int64_t kv_len,
+                bool direct, int num_splits, int64_t ws_bytes) {
+  if (is_causal != 0) return true;
+  const int64_t qblocks = batch * q_heads * cdiv(q_len, w4::kBM);
+  if (qblocks <= 0 || qblocks > device_cus()) return false;
+  const w4::SplitPlan sp = w4::plan_splits(!direct, qblocks, kv_len, head_dim, false, num_splits, ws_bytes);
+  return sp.nfull + (qblocks - sp.nfull) * sp.nsplit <= device_cus() &&
+         cdiv(kv_len, w4::kBN) >= kMinGroupTiles * sp.nsplit;
 }
 
 }  // namespace sage
@@ -215,10 +253,12 @@ void* scratch_address(const char* fn) {
 // attn_fwd of the block shape the launch runs (the arguments include head_dim and is_causal again)
 template <typename... Args>
 int run_attn(int64_t head_dim, int is_causal, int64_t batch, int64_t q_heads, int64_t q_len, int64_t kv_len, int qk,
-             Args... args) {
+             int num_splits, int64_t ws_bytes, Args... args) {
   const bool direct = qk == w8::kQkF16 || qk == w8::kQkBf16 || qk == w8::kQkF16V;
-  return small_blocks(head_dim, is_causal, batch, q_heads, q_len, kv_len, direct) ? w4::attn_fwd(qk, args...)
-                                                                                  : w8::attn_fwd(qk, args...);
+  if (!small_blocks(head_dim, is_causal, batch, q_heads, q_len, kv_len, direct)) return w8::attn_fwd(qk, args...);
+  return key_groups(is_causal, head_dim, batch, q_heads, q_len, kv_len, direct, num_splits, ws_bytes)
+             ? g2::attn_fwd(qk, args...)
+             : w4::attn_fwd(qk, args...);
 }
 
 // The plan of the shape the launch runs and its workspace bytes (or a negative status).
@@ -247,7 +287,7 @@ extern "C" int sage_attn_i8_fwd(const int8_t* q_i8, const int8_t* k_i8, const vo
                                 int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_n,
                                 int is_causal, void* stream) {
   clear_error();
-  return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len, w8::kQkI8, q_i8, k_i8, value_t, out, nullptr,
+  return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len, w8::kQkI8, 1, 0, q_i8, k_i8, value_t, out, nullptr,
                   q_scale, k_scale, out_dtype, batch, q_heads, kv_heads, q_len, kv_len, head_dim,
                   q_heads * q_len * head_dim, q_len * head_dim, head_dim, kv_heads * kv_len * head_dim,
                   kv_len * head_dim, head_dim, 0, 0, 0, o_stride_b, o_stride_h, o_stride_n, is_causal, 0.0, 1, nullptr,
@@ -261,7 +301,7 @@ extern "C" int sage_attn_i8_fwd_lse(const int8_t* q_i8, const int8_t* k_i8, cons
                                     int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_n,
                                     int is_causal, void* stream) {
   clear_error();
-  return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len, w8::kQkI8, q_i8, k_i8, value_t, out, lse, q_scale,
+  return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len, w8::kQkI8, 1, 0, q_i8, k_i8, value_t, out, lse, q_scale,
                   k_scale, out_dtype, batch, q_heads, kv_heads, q_len, kv_len, head_dim, q_heads * q_len * head_dim,
                   q_len * head_dim, head_dim, kv_heads * kv_len * head_dim, kv_len * head_dim, head_dim, 0, 0, 0,
                   o_stride_b, o_stride_h, o_stride_n, is_causal, 0.0, 1, nullptr, 0, stream, "sage_attn_i8_fwd_lse");
@@ -277,7 +317,8 @@ extern "C" int sage_attn_direct_fwd(const void* query, const void* key, const vo
                                     int64_t workspace_bytes, void* stream) {
   clear_error();
   return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len,
-                  dtype == SAGE_DTYPE_BF16 ? w8::kQkBf16 : w8::kQkF16, query, key, value_t, out, lse, nullptr, nullptr,
+                  dtype == SAGE_DTYPE_BF16 ? w8::kQkBf16 : w8::kQkF16, num_splits,
+                  workspace != nullptr ? workspace_bytes : 0, query, key, value_t, out, lse, nullptr, nullptr,
                   dtype, batch, q_heads, kv_heads, q_len, kv_len, head_dim, q_stride_b, q_stride_h, q_stride_n,
                   k_stride_b, k_stride_h, k_stride_n, 0, 0, 0, o_stride_b, o_stride_h, o_stride_n, is_causal, sm_scale,
                   num_splits, workspace, workspace_bytes, stream, "sage_attn_direct_fwd");
@@ -293,7 +334,8 @@ extern "C" int sage_attn_direct_fwd_vrows(const void* query, const void* key, co
                                           int is_causal, double sm_scale, int num_splits, void* workspace,
                                           int64_t workspace_bytes, void* stream) {
   clear_error();
-  return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len, w8::kQkF16V, query, key, value, out, lse, nullptr,
+  return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len, w8::kQkF16V, num_splits,
+                  workspace != nullptr ? workspace_bytes : 0, query, key, value, out, lse, nullptr,
                   nullptr, dtype, batch, q_heads, kv_heads, q_len, kv_len, head_dim, q_stride_b, q_stride_h,
                   q_stride_n, k_stride_b, k_stride_h, k_stride_n, v_stride_b, v_stride_h, v_stride_n, o_stride_b,
                   o_stride_h, o_stride_n, is_causal, sm_scale, num_splits, workspace, workspace_bytes, stream,
@@ -309,7 +351,8 @@ extern "C" int sage_attn_i8_fwd_qfused(const void* query, const int8_t* k_i8, co
                                        int is_causal, double sm_scale, int num_splits, void* workspace,
                                        int64_t workspace_bytes, void* stream) {
   clear_error();
-  return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len, w8::kQkI8F, query, k_i8, value_t, out, lse,
+  return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len, w8::kQkI8F, num_splits,
+                  workspace != nullptr ? workspace_bytes : 0, query, k_i8, value_t, out, lse,
                   nullptr, k_scale, dtype, batch, q_heads, kv_heads, q_len, kv_len, head_dim, q_stride_b, q_stride_h,
                   q_stride_n, kv_heads * kv_len * head_dim, kv_len * head_dim, head_dim, 0, 0, 0, o_stride_b,
                   o_stride_h, o_stride_n, is_causal, sm_scale, num_splits, workspace, workspace_bytes, stream,
@@ -326,7 +369,8 @@ extern "C" int sage_attn_i8_fwd_qfused_vrows(const void* query, const int8_t* k_
                                              int is_causal, double sm_scale, int num_splits, void* workspace,
                                              int64_t workspace_bytes, void* stream) {
   clear_error();
-  return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len, w8::kQkI8FV, query, k_i8, value, out, lse,
+  return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len, w8::kQkI8FV, num_splits,
+                  workspace != nullptr ? workspace_bytes : 0, query, k_i8, value, out, lse,
                   nullptr, k_scale, dtype, batch, q_heads, kv_heads, q_len, kv_len, head_dim, q_stride_b, q_stride_h,
                   q_stride_n, kv_heads * kv_len * head_dim, kv_len * head_dim, head_dim, v_stride_b, v_stride_h,
                   v_stride_n, o_stride_b, o_stride_h, o_stride_n, is_causal, sm_scale, num_splits, workspace,
@@ -359,7 +403,8 @@ extern "C" int sage_attn_i8_fwd_qfused_noalloc(const void* query, const int8_t* 
     ws = scratch_address(fn);
     if (ws == nullptr) return SAGE_ERR_HIP;
   }
-  return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len, w8::kQkI8F, query, k_i8, value_t, out, lse,
+  return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len, w8::kQkI8F, num_splits,
+                  ws != nullptr ? kScratchBytes : 0, query, k_i8, value_t, out, lse,
                   nullptr, k_scale, dtype, batch, q_heads, kv_heads, q_len, kv_len, head_dim, q_stride_b, q_stride_h,
                   q_stride_n, kv_heads * kv_len * head_dim, kv_len * head_dim, head_dim, 0, 0, 0, o_stride_b,
                   o_stride_h, o_stride_n, is_causal, sm_scale, num_splits, ws, ws != nullptr ? kScratchBytes : 0,
