@@ -60,35 +60,9 @@
 #include <type_traits>
 #include <utility>
 
-#include "sage_common.h"
+#include "attn_device.h"
 
 namespace sage {
-namespace {
-
-// Compute units of the current device, read once per device (256, the
-// MI355X count, if the runtime cannot tell).
-int device_cus() {
-  constexpr int kDevs = 64;
-  static std::atomic<int> cache[kDevs];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0) {
-    (void)hipGetLastError();
-    return 256;
-  }
-  if (dev < kDevs) {
-    const int v = cache[dev].load(std::memory_order_relaxed);
-    if (v > 0) return v;
-  }
-  int v = 0;
-  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) {
-    (void)hipGetLastError();
-    v = 256;
-  }
-  if (dev < kDevs) cache[dev].store(v, std::memory_order_relaxed);
-  return v;
-}
-
-}  // namespace
 
 // The kernels and their host code in three block shapes (attn_body.inc):
 //   * w8: 8 waves x 32 query rows = 256-row q-blocks, one block per CU;

@@ -91,13 +91,15 @@ at::Tensor split_workspace(bool quantized, const Dims& q, int64_t kv_len, bool c
 
 void* ptr(const at::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
-// Direct path, fp16 inputs: V is read in place (sage_attn_direct_fwd_vrows)
-// instead of through a V_T pass wherever that measured faster on MI355X
-// (whole direct call, launches queued): every D = 128 length of the direct
-// range (kv 77 -16%, 1024 -4% to -15%, 2048 -2.5% to -7%) and D = 64 up to
-// this many keys (kv 77 -10% to -19%, 1024 -4%, 1280 -2%; 1536 +5%, 3072 causal
-// +9%: the in-place V operand takes twice the LDS reads per P.V MFMA).
-constexpr int64_t kVRowsMaxKeysD64 = 1280;
+// INT8 path, fp16 inputs: V is read in place (sage_attn_i8_fwd_qfused_vrows,
+// the same output bit for bit) instead of through a V_T pass up to this many
+// query rows per kv head.  The pass saved is proportional to the V of a head,
+// the cost (twice the LDS reads per P.V MFMA) to its V times the query rows
+// that read it.  Whole call on MI355X, V_T / in place: B1 H16 S4096 D128 causal
+// 85.6 / 79.2 us, non-causal 118.1 / 114.8; B1 H8 S7000 D64 causal 69.8 / 67.4;
+// B1 H10 S4096 D64 61.1 / 60.0; S9216 D64 and D128 0-1% faster; Hq32 Hkv8
+// S16384 D128 causal (65536 rows) 1554 / 1566.
+constexpr int64_t kVRowsMaxQueries = 8192;
 
 py::object sageattn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, int64_t layout, bool is_causal, double sm_scale,
                         bool return_lse, bool smooth_k, bool direct, int64_t num_splits, int64_t stream_handle) {
@@ -136,8 +138,10 @@ py::object sageattn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, int64_t layout
     }
     int64_t ws_bytes = 0;
     at::Tensor ws = split_workspace(false, qd, Sk, is_causal, num_splits, q, &ws_bytes);
-    if (dtype == SAGE_DTYPE_F16 && vd.sn >= D && (D == 128 || Sk <= kVRowsMaxKeysD64)) {
-      // fp16 V read in place: one launch, the same output bit for bit as the V_T path below
+    if (dtype == SAGE_DTYPE_F16 && vd.sn >= D && (Sk + 5 * SAGE_VT_ALIGN) * vd.sn * 2 <= UINT32_MAX) {
+      // fp16 V read in place: one launch, the same output bit for bit as the V_T path below.  Whole call on MI355X,
+      // V_T / in place: D64 causal B1 H32 S2048 37.5 / 29.8 us, H20 S3072 50.4 / 43.6, H16 S6144 142 / 133; D64
+      // non-causal B1 H20 S1536 23.9 / 19.8, S2304 43.8 / 39.8
       check("sage_attn_direct_fwd_vrows",
             sage_attn_direct_fwd_vrows(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                                        static_cast<float*>(ptr(lse)), dtype, B, Hq, Hkv, Sq, Sk, D, qd.sb, qd.sh,
@@ -160,11 +164,17 @@ py::object sageattn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, int64_t layout
     // the attention kernel (the q_int8 and q_scale of quant_qk_int8, so the
     // same output, without the int8 Q round trip).  smooth_k: K minus its mean
     // (reference mean_seq, csrc/attn_gfx11.cu:1937-1972), the mean's chunk
-    // sums in a launch before, finished by the quantisation blocks
+    // sums in a launch before, finished by the quantisation blocks.  fp16 V
+    // with few enough query rows stays where it is: K quantisation alone, and
+    // the kernel that reads V in place
+    const bool smooth = smooth_k && Sk > 0;
+    const bool v_rows = dtype == SAGE_DTYPE_F16 && !smooth && vd.sn >= D && Hq / Hkv * Sq <= kVRowsMaxQueries &&
+                        (Sk + 5 * SAGE_VT_ALIGN) * vd.sn * 2 <= UINT32_MAX;
     at::Tensor k8 = at::empty({B, Hkv, Sk, D}, q.options().dtype(at::kChar));
     at::Tensor ks = at::empty({B, Hkv, (Sk + SAGE_K_GROUP - 1) / SAGE_K_GROUP}, q.options().dtype(at::kFloat));
-    at::Tensor vt = at::empty({B, Hkv, D, np}, q.options().dtype(at::kHalf));
-    if (smooth_k && Sk > 0) {
+    at::Tensor vt;
+    if (!v_rows) vt = at::empty({B, Hkv, D, np}, q.options().dtype(at::kHalf));
+    if (smooth) {
       const int64_t mb = sage_k_mean_workspace_bytes(B, Hkv, Sk, D);
       if (mb < 0) check("sage_k_mean_workspace_bytes", static_cast<int>(mb));
       at::Tensor mws = at::empty({(std::max<int64_t>(mb, 4) + 3) / 4}, q.options().dtype(at::kFloat));
@@ -173,6 +183,11 @@ py::object sageattn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, int64_t layout
                                    static_cast<int8_t*>(k8.data_ptr()), static_cast<float*>(ks.data_ptr()),
                                    vt.data_ptr(), dtype, B, Hkv, Sk, D, kd.sb, kd.sh, kd.sn, vd.sb, vd.sh, vd.sn,
                                    stream));
+    } else if (v_rows) {
+      check("sage_quant_qk_i8",
+            sage_quant_qk_i8(nullptr, k.data_ptr(), nullptr, nullptr, nullptr, static_cast<int8_t*>(k8.data_ptr()),
+                             static_cast<float*>(ks.data_ptr()), dtype, B, Hkv, Hkv, 0, Sk, D, 0, 0, 0, kd.sb, kd.sh,
+                             kd.sn, 1.0, stream));
     } else {
       check("sage_prep_kv_i8",
             sage_prep_kv_i8(k.data_ptr(), v.data_ptr(), nullptr, static_cast<int8_t*>(k8.data_ptr()),
@@ -183,12 +198,22 @@ py::object sageattn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, int64_t layout
     // the fused kernel writes the real log-sum-exp of each row
     int64_t ws_bytes = 0;
     at::Tensor ws = split_workspace(true, qd, Sk, is_causal, num_splits, q, &ws_bytes);
-    check("sage_attn_i8_fwd_qfused",
-          sage_attn_i8_fwd_qfused(q.data_ptr(), static_cast<const int8_t*>(k8.data_ptr()), vt.data_ptr(),
-                                  o.data_ptr(), static_cast<float*>(ptr(lse)), static_cast<const float*>(ks.data_ptr()),
-                                  dtype, B, Hq, Hkv, Sq, Sk, D, qd.sb, qd.sh, qd.sn, od.sb, od.sh, od.sn,
-                                  is_causal ? 1 : 0, sm_scale, static_cast<int>(num_splits), ptr(ws), ws_bytes,
-                                  stream));
+    if (v_rows) {
+      check("sage_attn_i8_fwd_qfused_vrows",
+            sage_attn_i8_fwd_qfused_vrows(q.data_ptr(), static_cast<const int8_t*>(k8.data_ptr()), v.data_ptr(),
+                                          o.data_ptr(), static_cast<float*>(ptr(lse)),
+                                          static_cast<const float*>(ks.data_ptr()), dtype, B, Hq, Hkv, Sq, Sk, D,
+                                          qd.sb, qd.sh, qd.sn, vd.sb, vd.sh, vd.sn, od.sb, od.sh, od.sn,
+                                          is_causal ? 1 : 0, sm_scale, static_cast<int>(num_splits), ptr(ws), ws_bytes,
+                                          stream));
+    } else {
+      check("sage_attn_i8_fwd_qfused",
+            sage_attn_i8_fwd_qfused(q.data_ptr(), static_cast<const int8_t*>(k8.data_ptr()), vt.data_ptr(),
+                                    o.data_ptr(), static_cast<float*>(ptr(lse)),
+                                    static_cast<const float*>(ks.data_ptr()), dtype, B, Hq, Hkv, Sq, Sk, D, qd.sb,
+                                    qd.sh, qd.sn, od.sb, od.sh, od.sn, is_causal ? 1 : 0, sm_scale,
+                                    static_cast<int>(num_splits), ptr(ws), ws_bytes, stream));
+    }
   }
   if (return_lse) return py::make_tuple(o, lse);
   return py::cast(o);
