@@ -332,6 +332,29 @@ int sage_attn_direct_fwd_vrows(const void* query, const void* key, const void* v
                                int is_causal, double sm_scale, int num_splits, void* workspace,
                                int64_t workspace_bytes, void* stream);
 
+/* Attention of few queries over a long key range, in one launch (two with key
+ * splits) on the caller's Q, K and V: non-causal, any grouping; quantized != 0
+ * computes the INT8 path (Q and K quantised inside the kernel, the values and
+ * scales of sage_quant_qk_i8, no K mean), 0 the direct fp16/bf16 path.  lse
+ * (or NULL) receives the rows' log-sum-exp.  K and V rows must not overlap and
+ * all strides be multiples of 8 elements, as q_len <= SAGE_FEW_MAX_ROWS and
+ * kv_len > 0.  workspace: sage_attn_few_workspace_bytes (0 when the launch
+ * runs unsplit).  Same outputs within rounding as the launches it stands for:
+ * sage_prep_kv_i8 + sage_attn_i8_fwd_qfused, or sage_v_layout +
+ * sage_attn_direct_fwd (csrc/attn_gfx11.cu:409-825, :1465-1885).
+ */
+#define SAGE_FEW_MAX_ROWS 4096
+int64_t sage_attn_few_workspace_bytes(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t q_len,
+                                      int64_t kv_len, int64_t head_dim);
+int sage_attn_few_fwd(int quantized, const void* query, const void* key, const void* value, void* out, float* lse,
+                      int dtype, int64_t batch, int64_t q_heads, int64_t kv_heads,
+                      int64_t q_len, int64_t kv_len, int64_t head_dim,
+                      int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
+                      int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n,
+                      int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_n,
+                      int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_n,
+                      double sm_scale, void* workspace, int64_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -13,7 +13,7 @@ Flags:
     compile: no packed fp32 VALU instructions are generated;
   * ``-ffp-contract=off`` on the prologue (its quantiser is bit-exact IEEE
     fp32 and must not fuse multiply-adds); no ``-ffast-math`` anywhere;
-  * ``-mllvm -amdgpu-mfma-vgpr-form`` on the attention kernel (MFMA
+  * ``-mllvm -amdgpu-mfma-vgpr-form`` on the attention kernels (MFMA
     accumulators in arch VGPRs, no per-tile AGPR copies).
 """
 from __future__ import annotations
@@ -58,6 +58,7 @@ SOURCES = [
     # MFMA results in arch VGPRs: the softmax reads every S element and the
     # rare O rescale touches O; AGPR residency costs v_accvgpr copies per tile
     ("attn.hip", ["-mllvm", "-amdgpu-mfma-vgpr-form"]),
+    ("attn_few.hip", ["-mllvm", "-amdgpu-mfma-vgpr-form"]),
 ]
 
 

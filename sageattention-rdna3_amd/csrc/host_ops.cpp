@@ -101,6 +101,33 @@ void* ptr(const at::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 // S16384 D128 causal (65536 rows) 1554 / 1566.
 constexpr int64_t kVRowsMaxQueries = 8192;
 
+// Few query rows per kv head against the key range: one pass over K and V in
+// place for the rows of all its query heads (sage_attn_few_fwd).  The general
+// path quantises K and transposes V first (INT8), pads each query head to 128
+// or 256 rows and reads K/V once per query head.  The rows are packed into
+// 32-row tiles; a launch of many tiles re-reads K/V per two of them.  Whole
+// call on MI355X, general / few: INT8, one tile: B8 Hq32 Hkv8 Sq1 Sk8192 D128
+// 225 / 55 us, B4 Hq32 Hkv4 Sq8 Sk16384 204 / 46; 4 tiles: B4 H16 Sq128 Sk4096
+// 66 / 39, H8 Sk8192 D64 26.6 / 23.9; 8 tiles: B1 H8 Sq256 Sk8192 D128 42 / 36,
+// D64 29.2 / 25.4; 16 tiles: 46 / 53, 32 / 34.  Direct: one tile B8 H8 Sq2
+// Sk4096 D64 34 / 17; 3 tiles H16 Sk2048 D128 19.5 / 18.5, H16 Sk1024 D64 12.4 /
+// 12.0; 4 tiles of 128-row heads 20.4 / 22.1; 8 tiles of 40-row heads (B2 Hq32
+// Hkv8 Sk3000) 39 / 22.
+constexpr int64_t kFewMaxTiles = 8;
+constexpr int64_t kFewMaxTilesDirect = 3;   // direct path, heads of more than kFewShortHead rows
+constexpr int64_t kFewShortHead = 64;
+
+bool few_queries(const Dims& q, const Dims& k, const Dims& v, bool direct) {
+  if (q.n <= 0 || k.n <= 0 || q.n > 32 * kFewMaxTiles) return false;
+  const int64_t units = q.h / k.h * ((q.n + 31) / 32);  // 32-token groups of the heads, never cut by a tile
+  const int64_t per_tile = 32 / std::min<int64_t>(q.n, 32);
+  const int64_t tiles = (units + per_tile - 1) / per_tile;
+  if (tiles > (direct && q.n > kFewShortHead ? kFewMaxTilesDirect : kFewMaxTiles)) return false;
+  constexpr int64_t kPastEnd = 24 * 32;  // keys past the last that the kernel's loads address (they read as zero)
+  return k.sn >= q.d && v.sn >= q.d && (k.n + kPastEnd) * k.sn * 2 <= UINT32_MAX &&
+         (k.n + kPastEnd) * v.sn * 2 <= UINT32_MAX && q.b * q.h <= INT32_MAX / SAGE_FEW_MAX_ROWS;
+}
+
 py::object sageattn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, int64_t layout, bool is_causal, double sm_scale,
                         bool return_lse, bool smooth_k, bool direct, int64_t num_splits, int64_t stream_handle) {
   if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4) throw py::value_error("q, k and v must be 4-D tensors");
@@ -130,7 +157,17 @@ py::object sageattn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, int64_t layout
   at::Tensor lse;
   if (return_lse) lse = at::empty({B, Hq, Sq}, q.options().dtype(at::kFloat));
 
-  if (direct) {
+  if (!is_causal && num_splits == 0 && !(smooth_k && !direct) && few_queries(qd, kd, vd, direct)) {
+    const int64_t ws_bytes = sage_attn_few_workspace_bytes(B, Hq, Hkv, Sq, Sk, D);
+    if (ws_bytes < 0) check("sage_attn_few_workspace_bytes", static_cast<int>(ws_bytes));
+    at::Tensor ws;
+    if (ws_bytes > 0) ws = at::empty({ws_bytes}, q.options().dtype(at::kByte));
+    check("sage_attn_few_fwd",
+          sage_attn_few_fwd(direct ? 0 : 1, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+                            static_cast<float*>(ptr(lse)), dtype, B, Hq, Hkv, Sq, Sk, D, qd.sb, qd.sh, qd.sn, kd.sb,
+                            kd.sh, kd.sn, vd.sb, vd.sh, vd.sn, od.sb, od.sh, od.sn, sm_scale, ptr(ws), ws_bytes,
+                            stream));
+  } else if (direct) {
     // the direct kernel reads Q and K in place (core.py:141-164); K rows must not overlap
     if (kd.sn < D) {
       k = k.contiguous();
