@@ -332,6 +332,21 @@ int sage_attn_direct_fwd_vrows(const void* query, const void* key, const void* v
                                int is_causal, double sm_scale, int num_splits, void* workspace,
                                int64_t workspace_bytes, void* stream);
 
+/*
+ * sage_attn_direct_fwd_vrows for bf16 inputs: `value` is the caller's bf16 V,
+ * read in place; the kernel converts its tiles to fp16 in LDS (round to nearest
+ * even, as sage_v_layout does), so results equal sage_v_layout +
+ * sage_attn_direct_fwd bit for bit.  Query, key, value and out are bf16.
+ */
+int sage_attn_direct_fwd_vrows_bf16(const void* query, const void* key, const void* value, void* out, float* lse,
+                                    int64_t batch, int64_t q_heads, int64_t kv_heads,
+                                    int64_t q_len, int64_t kv_len, int64_t head_dim,
+                                    int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
+                                    int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n,
+                                    int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_n,
+                                    int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_n,
+                                    int is_causal, double sm_scale, int num_splits, void* workspace,
+                                    int64_t workspace_bytes, void* stream);
 /* Attention of few queries over a long key range, in one launch (two with key
  * splits) on the caller's Q, K and V: non-causal, any grouping; quantized != 0
  * computes the INT8 path (Q and K quantised inside the kernel, the values and

@@ -228,7 +228,7 @@ void* scratch_address(const char* fn) {
 template <typename... Args>
 int run_attn(int64_t head_dim, int is_causal, int64_t batch, int64_t q_heads, int64_t q_len, int64_t kv_len, int qk,
              int num_splits, int64_t ws_bytes, Args... args) {
-  const bool direct = qk == w8::kQkF16 || qk == w8::kQkBf16 || qk == w8::kQkF16V;
+  const bool direct = qk == w8::kQkF16 || qk == w8::kQkBf16 || qk == w8::kQkF16V || qk == w8::kQkBf16V;
   if (!small_blocks(head_dim, is_causal, batch, q_heads, q_len, kv_len, direct)) return w8::attn_fwd(qk, args...);
   return key_groups(is_causal, head_dim, batch, q_heads, q_len, kv_len, direct, num_splits, ws_bytes)
              ? g2::attn_fwd(qk, args...)
@@ -349,6 +349,24 @@ extern "C" int sage_attn_i8_fwd_qfused_vrows(const void* query, const int8_t* k_
                   q_stride_n, kv_heads * kv_len * head_dim, kv_len * head_dim, head_dim, v_stride_b, v_stride_h,
                   v_stride_n, o_stride_b, o_stride_h, o_stride_n, is_causal, sm_scale, num_splits, workspace,
                   workspace_bytes, stream, "sage_attn_i8_fwd_qfused_vrows");
+}
+
+extern "C" int sage_attn_direct_fwd_vrows_bf16(const void* query, const void* key, const void* value, void* out,
+                                               float* lse, int64_t batch, int64_t q_heads, int64_t kv_heads,
+                                               int64_t q_len, int64_t kv_len, int64_t head_dim,
+                                               int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_n,
+                                               int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_n,
+                                               int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_n,
+                                               int64_t o_stride_b, int64_t o_stride_h, int64_t o_stride_n,
+                                               int is_causal, double sm_scale, int num_splits, void* workspace,
+                                               int64_t workspace_bytes, void* stream) {
+  clear_error();
+  return run_attn(head_dim, is_causal, batch, q_heads, q_len, kv_len, w8::kQkBf16V, num_splits,
+                  workspace != nullptr ? workspace_bytes : 0, query, key, value, out, lse, nullptr,
+                  nullptr, SAGE_DTYPE_BF16, batch, q_heads, kv_heads, q_len, kv_len, head_dim, q_stride_b, q_stride_h,
+                  q_stride_n, k_stride_b, k_stride_h, k_stride_n, v_stride_b, v_stride_h, v_stride_n, o_stride_b,
+                  o_stride_h, o_stride_n, is_causal, sm_scale, num_splits, workspace, workspace_bytes, stream,
+                  "sage_attn_direct_fwd_vrows_bf16");
 }
 
 extern "C" int sage_attn_i8_fwd_qfused_noalloc(const void* query, const int8_t* k_i8, const void* value_t, void* out,

@@ -175,10 +175,20 @@ py::object sageattn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, int64_t layout
     }
     int64_t ws_bytes = 0;
     at::Tensor ws = split_workspace(false, qd, Sk, is_causal, num_splits, q, &ws_bytes);
-    if (dtype == SAGE_DTYPE_F16 && vd.sn >= D && (Sk + 5 * SAGE_VT_ALIGN) * vd.sn * 2 <= UINT32_MAX) {
-      // fp16 V read in place: one launch, the same output bit for bit as the V_T path below.  Whole call on MI355X,
-      // V_T / in place: D64 causal B1 H32 S2048 37.5 / 29.8 us, H20 S3072 50.4 / 43.6, H16 S6144 142 / 133; D64
-      // non-causal B1 H20 S1536 23.9 / 19.8, S2304 43.8 / 39.8
+    // V read in place: one launch, the same output bit for bit as the V_T path (kept for V rows that overlap or
+    // span more than 32-bit offsets).  Whole call on MI355X, V_T / in place: fp16 D64 causal B1 H32 S2048 37.5 / 29.8
+    // us, H20 S3072 50.4 / 43.6, H16 S6144 142 / 133; D64 non-causal B1 H20 S1536 23.9 / 19.8, S2304 43.8 / 39.8;
+    // bf16 D128 B1 H16 Sq4096 kv512 27.9 / 25.0, kv154 19.9 / 16.6, causal H32 S2048 58.4 / 52.0, H8 S1024 22.4 /
+    // 21.6, B2 H32 S2048 152 / 150; bf16 D64 H20 S1024 17.2 / 14.7, causal H16 S6144 147.8 / 143.3
+    const bool v_rows = vd.sn >= D && (Sk + 5 * SAGE_VT_ALIGN) * vd.sn * 2 <= UINT32_MAX;
+    if (v_rows && dtype == SAGE_DTYPE_BF16) {
+      check("sage_attn_direct_fwd_vrows_bf16",
+            sage_attn_direct_fwd_vrows_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+                                            static_cast<float*>(ptr(lse)), B, Hq, Hkv, Sq, Sk, D, qd.sb, qd.sh, qd.sn,
+                                            kd.sb, kd.sh, kd.sn, vd.sb, vd.sh, vd.sn, od.sb, od.sh, od.sn,
+                                            is_causal ? 1 : 0, sm_scale, static_cast<int>(num_splits), ptr(ws),
+                                            ws_bytes, stream));
+    } else if (v_rows && dtype == SAGE_DTYPE_F16) {
       check("sage_attn_direct_fwd_vrows",
             sage_attn_direct_fwd_vrows(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                                        static_cast<float*>(ptr(lse)), dtype, B, Hq, Hkv, Sq, Sk, D, qd.sb, qd.sh,

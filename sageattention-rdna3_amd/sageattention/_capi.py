@@ -80,6 +80,10 @@ SIGNATURES = {
                                         _I64, _I64, _I64, _I64, _I64, _I64,
                                         _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
                                         _I, ctypes.c_double, _I, _P, _I64, _P]),
+    "sage_attn_direct_fwd_vrows_bf16": (_I, [_P, _P, _P, _P, _P,
+                                             _I64, _I64, _I64, _I64, _I64, _I64,
+                                             _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
+                                             _I, ctypes.c_double, _I, _P, _I64, _P]),
     "sage_attn_few_workspace_bytes": (_I64, [_I64, _I64, _I64, _I64, _I64, _I64]),
     "sage_attn_few_fwd": (_I, [_I, _P, _P, _P, _P, _P, _I,
                                _I64, _I64, _I64, _I64, _I64, _I64,

@@ -1,0 +1,64 @@
+"""bf16 V read in place (converted to fp16 in LDS) by the direct kernel against the V_T path, bit for bit, through the
+C ABI: the three block shapes (256-row, 128-row, two key groups), ring depths, ragged ends, one tile, key
+splits, causal and not, grouped heads, a strided V; values that overflow fp16 become infinite on both paths."""
+import pytest
+import torch
+
+from _helpers import Config, make_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def case(B, Hq, Hkv, Sq, S, D, layout, causal):
+    return Config(f"B{B}H{Hq}k{Hkv}q{Sq}kv{S}D{D}_{layout}{'_c' if causal else ''}", B, Hq, Hkv, S, D, "bf16", layout,
+                  causal, False, Sq=None if Sq == S else Sq)
+
+
+CASES = [
+    case(1, 2, 2, 40, 1, 128, "HND", False),
+    case(1, 3, 1, 100, 65, 64, "NHD", False),
+    case(1, 4, 2, 300, 513, 128, "NHD", False),
+    case(1, 10, 10, 700, 154, 64, "NHD", False),
+    case(1, 5, 5, 900, 1100, 64, "HND", False),
+    case(2, 20, 20, 1000, 700, 64, "HND", False),
+    case(1, 6, 3, 777, 777, 128, "HND", True),
+    case(1, 3, 3, 130, 2000, 128, "NHD", True),
+    case(1, 7, 7, 1021, 1021, 64, "NHD", True),
+    case(1, 34, 34, 2300, 2300, 128, "HND", True),
+    case(1, 33, 33, 2100, 1300, 128, "HND", False),
+]
+
+
+@pytest.mark.parametrize("splits", [0, 1, 3])
+@pytest.mark.parametrize("cfg", CASES, ids=lambda c: c.name)
+def test_bf16_v_in_place_equals_vt_path(cfg, splits):
+    from sageattention import _capi, ops
+
+    print(f"[bf16 v rows] {cfg.name} splits={splits}", flush=True)
+    q, k, v = (t.cuda() for t in make_inputs(cfg, seed=11))
+    v.view(-1)[::1001] = 1e6  # past fp16's range
+    wide = torch.zeros(v.shape[:-1] + (2 * cfg.D,), device="cuda", dtype=v.dtype)
+    wide[..., 8: 8 + cfg.D] = v
+    v = wide[..., 8: 8 + cfg.D]
+    lay = ops.HND if cfg.layout == "HND" else ops.NHD
+    causal, sm = int(cfg.causal), cfg.D ** -0.5
+    vt = torch.empty(cfg.B, cfg.Hkv, cfg.D, (cfg.S + 63) // 64 * 64, device="cuda", dtype=torch.float16)
+    ops.v_transpose(v, vt, lay)
+    o_ref, o = torch.empty_like(q), torch.full_like(q, float("nan"))
+    lse_ref = torch.empty(cfg.B, cfg.Hq, cfg.q_len, device="cuda")
+    lse = torch.full_like(lse_ref, float("nan"))
+    sq, sk, sv, so = ([x.stride(0)] + ([x.stride(1), x.stride(2)] if lay == ops.HND else [x.stride(2), x.stride(1)])
+                      for x in (q, k, v, o))
+    ws_bytes = 0 if cfg.causal else _capi.query("sage_attn_workspace_bytes", 0, cfg.B, cfg.Hq, cfg.q_len,
+                                                cfg.S, cfg.D, 0, splits)
+    ws = torch.empty(max(ws_bytes, 16), device="cuda", dtype=torch.uint8)
+    sizes = (cfg.B, cfg.Hq, cfg.Hkv, cfg.q_len, cfg.S, cfg.D)
+    tail = (causal, sm, splits, ws.data_ptr() if ws_bytes else None, ws_bytes, ops._stream(q))
+    ops.bf16_attn_t(q, k, vt, o_ref, lay, causal, sm, 0, lse=lse_ref, num_splits=splits)
+    _capi.call("sage_attn_direct_fwd_vrows_bf16", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+               lse.data_ptr(), *sizes, *sq, *sk, *sv, *so, *tail)
+    torch.cuda.synchronize()
+    # infinities meet on both paths; where they cancel to NaN both must be NaN
+    assert torch.equal(torch.isnan(o), torch.isnan(o_ref))
+    assert torch.equal(torch.nan_to_num(o.float()), torch.nan_to_num(o_ref.float()))
+    assert torch.equal(lse, lse_ref)
