@@ -12,9 +12,12 @@
 // the stream handle the caller passes (the current stream of the tensors'
 // device), and torch allocates on that same stream, so temporaries released
 // here return to the caching allocator in stream order.
+#include <c10/core/impl/VirtualGuardImpl.h>
 #include <torch/extension.h>
 
+#include <cmath>
 #include <cstdint>
+#include <cstdlib>
 #include <sstream>
 #include <string>
 
@@ -266,6 +269,43 @@ py::object sageattn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, int64_t layout
   return py::cast(o);
 }
 
+// The reference's choice between the direct and the INT8 path with its default
+// thresholds (sageattention/core.py:113-139; core.use_direct_path has the
+// environment overrides too).
+bool default_direct(int64_t head_dim, int64_t q_len, int64_t kv_len, bool causal, bool hnd) {
+  if (head_dim == 64) {
+    if (causal || q_len < kv_len) return kv_len <= 6144;
+    return kv_len <= (hnd ? 2048 : 3072);
+  }
+  return kv_len <= (q_len * 2 < kv_len ? 4096 : 2048);
+}
+
+// The whole call where nothing is unusual: fp16/bf16 tensors that pass every
+// check of sageattn on the current device, and none of its environment
+// variables set.  None otherwise, and the Python function goes through its
+// steps (and raises what fails).  Those steps cost 3.5 us a call, as much as
+// the launches of the short calls; these checks 0.3 us.
+py::object sageattn_plain(at::Tensor q, at::Tensor k, at::Tensor v, bool hnd, bool is_causal,
+                          std::optional<double> sm_scale, bool return_lse, bool smooth_k, int64_t stream_handle) {
+  const auto dt = q.scalar_type();
+  if ((dt != at::kHalf && dt != at::kBFloat16) || k.scalar_type() != dt || v.scalar_type() != dt || !q.is_cuda() ||
+      k.device() != q.device() || v.device() != q.device() || q.dim() != 4 || k.dim() != 4 || v.dim() != 4)
+    return py::none();
+  const int64_t d = q.size(3);
+  if ((d != 64 && d != 128) || q.stride(3) != 1 || k.stride(3) != 1 || v.stride(3) != 1 || q.stride(0) % 8 != 0 ||
+      q.stride(1) % 8 != 0 || q.stride(2) % 8 != 0)
+    return py::none();
+  for (const char* name :
+       {"SAGEATTN_KV_SPLITS", "SAGEATTN_DIRECT_THRESHOLD_D64", "SAGEATTN_DIRECT_THRESHOLD_D64_CAUSAL",
+        "SAGEATTN_DIRECT_THRESHOLD_D64_CROSS", "SAGEATTN_DIRECT_THRESHOLD_D128", "SAGEATTN_DIRECT_THRESHOLD_D128_CROSS"})
+    if (std::getenv(name) != nullptr) return py::none();
+  if (c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getDevice().index() != q.device().index()) return py::none();
+  const int seq = hnd ? 2 : 1;
+  const bool direct = default_direct(d, q.size(seq), k.size(seq), is_causal, hnd);
+  return sageattn_fwd(q, k, v, hnd ? 1 : 0, is_causal, sm_scale ? *sm_scale : std::pow(static_cast<double>(d), -0.5),
+                      return_lse, smooth_k, direct, 0, stream_handle);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -279,6 +319,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sageattn_fwd", &sageattn_fwd, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("tensor_layout"),
         py::arg("is_causal"), py::arg("sm_scale"), py::arg("return_lse"), py::arg("smooth_k"), py::arg("direct"),
         py::arg("num_splits"), py::arg("stream"));
+  m.def("sageattn_plain", &sageattn_plain, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("hnd"),
+        py::arg("is_causal"), py::arg("sm_scale"), py::arg("return_lse"), py::arg("smooth_k"), py::arg("stream"));
+  m.def("default_direct", &default_direct, py::arg("head_dim"), py::arg("q_len"), py::arg("kv_len"),
+        py::arg("is_causal"), py::arg("hnd"));
   py::register_exception_translator([](std::exception_ptr p) {
     try {
       if (p) std::rethrow_exception(p);

@@ -91,6 +91,16 @@ def sageattn(
     ``bm_sel`` (the reference's experimental direct-kernel tile override) is
     accepted and ignored; other unknown kwargs are ignored too.
     """
+    # the common call in one compiled step; None where a check or an override needs the steps below
+    if (type(q) is torch.Tensor and type(k) is torch.Tensor and type(v) is torch.Tensor and q.is_cuda
+            and tensor_layout in ("HND", "NHD") and (sm_scale is None or type(sm_scale) is float)
+            and ops._raw_stream is not None):
+        res = (_host_mod or _host()).sageattn_plain(
+            q, k, v, tensor_layout == "HND", bool(is_causal), sm_scale, bool(return_lse),
+            bool(kwargs.get("smooth_k", False)), ops._raw_stream(q.get_device()))
+        if res is not None:
+            return res
+
     dtype = q.dtype
     assert q.is_cuda, "Input tensors must be on CUDA/HIP device."
     assert dtype in [torch.float16, torch.bfloat16, torch.float32], (
