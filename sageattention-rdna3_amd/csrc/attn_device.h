@@ -157,5 +157,32 @@ __device__ __forceinline__ float wave_max64(float v) {
   return xhalf_max(v);
 }
 
+// fl(x * s) rounded half away from zero.  round_half_away_i8 without its
+// clamp: x * s has a magnitude of at most 127 (1 + 2^-22) for finite x, as s =
+// fl(127 / max|x|) (times Q's pre-scale, which max|x| includes), and the
+// conversion turns NaN into 0.
+__device__ __forceinline__ int quant1(float x, float s) {
+#pragma clang fp contract(off)
+  const float t = x * s;
+  const float u = t + __builtin_copysignf(0.5f, t);
+  int r;
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(u));
+  return r;
+}
+
+// 16 elements (8 dwords) -> 16 int8 (the MFMA operand of a lane)
+template <bool BF16>
+__device__ __forceinline__ int4_t quant16(const uint32_t (&w)[8], float s) {
+  int4_t o;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float2_t a = unpack2<BF16>(w[2 * k]), b = unpack2<BF16>(w[2 * k + 1]);
+    const uint32_t lo = __builtin_amdgcn_perm(quant1(a.y, s), quant1(a.x, s), 0x0c0c0400u);
+    const uint32_t hi = __builtin_amdgcn_perm(quant1(b.y, s), quant1(b.x, s), 0x04000c0cu);
+    o[k] = static_cast<int>(lo | hi);
+  }
+  return o;
+}
+
 }  // namespace
 }  // namespace sage
