@@ -97,12 +97,14 @@ void* ptr(const at::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 // INT8 path, fp16 inputs: V is read in place (sage_attn_i8_fwd_qfused_vrows,
 // the same output bit for bit) instead of through a V_T pass up to this many
 // query rows per kv head.  The pass saved is proportional to the V of a head,
-// the cost (twice the LDS reads per P.V MFMA) to its V times the query rows
-// that read it.  Whole call on MI355X, V_T / in place: B1 H16 S4096 D128 causal
-// 85.6 / 79.2 us, non-causal 118.1 / 114.8; B1 H8 S7000 D64 causal 69.8 / 67.4;
-// B1 H10 S4096 D64 61.1 / 60.0; S9216 D64 and D128 0-1% faster; Hq32 Hkv8
-// S16384 D128 causal (65536 rows) 1554 / 1566.
-constexpr int64_t kVRowsMaxQueries = 8192;
+// the cost (twice the LDS reads per P.V MFMA, ~3% of the kernel) to its V times
+// the query rows that read it.  Whole call on MI355X, V_T / in place: B1 H16
+// S4096 D128 causal 85.6 / 79.2 us, non-causal 118.1 / 114.8; B1 H8 S7000 D64
+// causal 69.8 / 67.4; B1 H10 S4096 D64 61.1 / 60.0; H24 S6000 D64 226.0 /
+// 224.5; B1 H5 S7423 D128 149.6 / 151.2; Hq32 Hkv8 S16384 D128 causal (65536
+// rows) 1554 / 1566.
+constexpr int64_t kVRowsMaxQueries = 6144;
+constexpr int64_t kVRowsMaxQueriesCausal = 8192;
 
 // Few query rows per kv head against the key range: one pass over K and V in
 // place for the rows of all its query heads (sage_attn_few_fwd).  The general
@@ -218,7 +220,8 @@ py::object sageattn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, int64_t layout
     // with few enough query rows stays where it is: K quantisation alone, and
     // the kernel that reads V in place
     const bool smooth = smooth_k && Sk > 0;
-    const bool v_rows = dtype == SAGE_DTYPE_F16 && !smooth && vd.sn >= D && Hq / Hkv * Sq <= kVRowsMaxQueries &&
+    const bool v_rows = dtype == SAGE_DTYPE_F16 && !smooth && vd.sn >= D &&
+                        Hq / Hkv * Sq <= (is_causal ? kVRowsMaxQueriesCausal : kVRowsMaxQueries) &&
                         (Sk + 5 * SAGE_VT_ALIGN) * vd.sn * 2 <= UINT32_MAX;
     at::Tensor k8 = at::empty({B, Hkv, Sk, D}, q.options().dtype(at::kChar));
     at::Tensor ks = at::empty({B, Hkv, (Sk + SAGE_K_GROUP - 1) / SAGE_K_GROUP}, q.options().dtype(at::kFloat));
