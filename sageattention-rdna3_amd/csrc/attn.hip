@@ -134,12 +134,14 @@ constexpr bool kSmallShape = true;
 constexpr double kLoneHalfBlockTileDirect = 0.70;
 constexpr double kLoneHalfBlockTileI8 = 0.77;
 
-// The shape a launch runs: w4 for D = 64 non-causal launches, and for causal
+// Whether a launch runs 128-row q-blocks (in w4 or g2, by key_groups): D = 64
+// non-causal launches, and causal ones.  The causal timings below compare the
+// 256-row blocks with 4-wave 128-row ones; g2 is faster still.  128 rows for causal
 // launches whose 256-row q-blocks would fill at most half the CUs (their
 // 128-row q-blocks then fill twice as many, one block per CU; B1 H8 S4096
 // D128 INT8: -27%; the D = 128 direct kernel, whose 98 KB of LDS fits once per
 // CU, at B1 H8/H16 S1024-2048: -27% to -32%); w8 for the rest (a causal launch
-// of 2048 +4% in w4).  A causal launch also runs w4 when its 256-row
+// of 2048 +4% in 128 rows).  A causal launch also runs 128 rows when its 256-row
 // q-blocks fill one round and the causal cost model rates the 128-row q-blocks
 // faster: with one block resident per CU they run as a persistent grid in
 // which the snake schedule gives each block a heavy and a light q-block.

@@ -72,3 +72,29 @@ def test_few_queries_strided_views_and_growing_scores(D, force_i8, monkeypatch):
         o, w = o.float().cpu().numpy(), w.float().cpu().numpy()
         assert np.all(np.abs(o - w) <= 2e-3 + 4e-3 * np.abs(w))
         assert torch.allclose(lse, wl, rtol=2e-6, atol=2e-4)
+
+
+@pytest.mark.parametrize("force_i8", [True, False])
+def test_few_queries_graph_capture_and_replay(force_i8, monkeypatch):
+    """The launches (attention, merge of the key splits) and the workspace in a HIP graph: every replay, with eager
+    work between, gives the eager call's bits."""
+    from sageattention import sageattn
+
+    monkeypatch.setenv("SAGEATTN_DIRECT_THRESHOLD_D128_CROSS", "-1" if force_i8 else "100000")
+    q, k, v = (t.cuda() for t in make_inputs(Config("few", 2, 8, 2, 6000, 128, "bf16", "HND", False, False, Sq=3), seed=9))
+    ref = sageattn(q, k, v)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        sageattn(q, k, v)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = sageattn(q, k, v)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)
+        assert torch.equal(sageattn(q, k, v), ref)
