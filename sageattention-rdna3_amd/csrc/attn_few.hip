@@ -30,6 +30,7 @@
 //   * the 4 waves' partial results merge in LDS; key splits (one block per CU
 //     in all) merge in a second small launch.
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 
 #include "attn_device.h"
@@ -230,7 +231,7 @@ __global__ __launch_bounds__(kFewThreads, 1) void few_attn_kernel(FewParams p) {
   float m_run[RT], l_run[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
-    m_run[rt] = -INFINITY;
+    m_run[rt] = -FLT_MAX;  // see the softmax: finite, so that a tile of -inf scores gives p = 0
     l_run[rt] = 0.0f;
 #pragma unroll
     for (int db = 0; db < C::kDB; ++db) o[rt][db] = float16_t_{};
@@ -359,12 +360,14 @@ __global__ __launch_bounds__(kFewThreads, 1) void few_attn_kernel(FewParams p) {
       for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(mx, y[r]);
       mx = xhalf_max(mx);
       // lazy reference max, as in attn_body.inc: it moves when a row's tile max
-      // passes it by more than kFewRescale, so p stays below 2^8
+      // passes it by more than kFewRescale, so p stays below 2^8.  It starts at
+      // the lowest finite value: a row whose scores are all -inf so far (keys
+      // masked through K) has p = exp2(-inf) = 0 against it, where -inf would
+      // give exp2(-inf + inf), and the first live score moves it
       if (__builtin_amdgcn_ballot_w64(mx > m_run[rt] + kFewRescale) != 0) {
         asm volatile("");  // a real branch
         float m_new = __builtin_fmaxf(m_run[rt], mx);
         if constexpr (I8) m_new = __builtin_ceilf(m_new);
-        m_new = (m_new == -INFINITY) ? 0.0f : m_new;
         const float alpha = fast_exp2(m_run[rt] - m_new);
         m_run[rt] = m_new;
         l_run[rt] *= alpha;
@@ -414,7 +417,7 @@ __global__ __launch_bounds__(kFewThreads, 1) void few_attn_kernel(FewParams p) {
 
   // ---- merge of the 4 waves: each hands over its O (unnormalised) and row
   // statistics, then merges a quarter of the 16-byte pieces of every row tile.
-  // A wave without tiles has l = 0 and m = -inf.
+  // A wave without tiles, or without a live key of the row, has l = 0.
   constexpr int kPieces = C::kDB * 4;  // float4 pieces per lane and row tile
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {

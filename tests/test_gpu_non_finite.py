@@ -1,0 +1,92 @@
+"""Infinite and NaN scores through ``sageattn``: keys masked through a channel of K (-inf, or bf16's lowest value against
+a query entry of 2, whose product overflows in fp32).  A masked key has weight 0 wherever it lies: whole key tiles, the
+first tiles that a wave, a key group or a key split reads, whole splits, all keys (output 0, LSE -inf).
+
+References: softmax attention in 64 bits over the same values (direct path), or the same call on the live keys alone
+(INT8 path; the masked ranges are whole scale groups, so the live keys quantise alike).  Tolerance: the parity tests'.
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = {"fp16": torch.float16, "bf16": torch.bfloat16}
+TOL = {"fp16": (2e-3, 4e-3), "bf16": (4e-3, 1.6e-2)}
+THRESHOLDS = ["SAGEATTN_DIRECT_THRESHOLD_" + n for n in ("D64", "D64_CAUSAL", "D64_CROSS", "D128", "D128_CROSS")]
+
+
+def set_path(monkeypatch, direct, splits=None):
+    for name in THRESHOLDS:
+        monkeypatch.setenv(name, "100000" if direct else "-1")
+    if splits is None:
+        monkeypatch.delenv("SAGEATTN_KV_SPLITS", raising=False)
+    else:
+        monkeypatch.setenv("SAGEATTN_KV_SPLITS", str(splits))
+
+
+def inputs(B, Hq, Hkv, Sq, Sk, D, dtype, low, seed=3):
+    """Small scores; channel 0 masks (q = 2 there, k = 0 for a live key), channel 1 shifts every score by -60 if low."""
+    g = torch.Generator().manual_seed(seed)
+    q, k, v = (torch.randn(B, h, s, D, generator=g) for h, s in ((Hq, Sq), (Hkv, Sk), (Hkv, Sk)))
+    q[..., :2], k[..., 0], k[..., 1] = torch.tensor([2.0, 1.0]), 0.0, -60.0 if low else 0.0
+    q[..., 2:] *= 0.3
+    return [x.to(DTYPES[dtype]).cuda() for x in (q, k, v)]
+
+
+def lowest(dtype):
+    return float("-inf") if dtype == "fp16" else torch.finfo(torch.bfloat16).min
+
+
+def exact(q, k, v, causal, scale=1.0):
+    """(output, LSE) in 64 bits; scores past fp32's range are infinite, a row without a live key gives 0 and -inf."""
+    B, Hq, Sq, D = q.shape
+    Sk, group = k.shape[2], Hq // k.shape[1]
+    out = torch.empty(B, Hq, Sq, D, dtype=torch.float64, device="cuda")
+    lse = torch.empty(B, Hq, Sq, dtype=torch.float64, device="cuda")
+    dead = torch.arange(Sk, device="cuda")[None] > torch.arange(Sq, device="cuda")[:, None]
+    for b in range(B):
+        for h in range(Hq):
+            s = (q[b, h].double() @ k[b, h // group].double().T * scale).float().double()
+            if causal:
+                s.masked_fill_(dead, float("-inf"))
+            m = s.amax(1, keepdim=True).clamp_min(torch.finfo(torch.float32).min)
+            p = (s - m).exp()
+            total = p.sum(1, keepdim=True)
+            out[b, h] = p @ v[b, h // group].half().double() / torch.where(total > 0, total, 1.0)
+            lse[b, h] = (m + total.log()).squeeze(1)
+    return out, lse
+
+
+def assert_close(got, want, dtype):
+    (o, lse), (w, wl) = got, want
+    atol, rtol = TOL[dtype]
+    assert torch.equal(torch.isnan(o), torch.isnan(w)) and torch.equal(torch.isnan(lse), torch.isnan(wl))
+    assert torch.allclose(o.double(), w.double(), atol=atol, rtol=rtol, equal_nan=True)
+    assert torch.allclose(lse.double(), wl.double(), atol=2e-4, rtol=2e-6, equal_nan=True)
+
+
+@pytest.mark.parametrize("low", [False, True])
+@pytest.mark.parametrize("masked", [(0, 40), (0, 129), (2048, 4096), (0, 4096)], ids=lambda m: f"keys{m[0]}-{m[1]}")
+@pytest.mark.parametrize("Sq", [4, 32], ids=["one_row_tile", "two_row_tiles"])
+@pytest.mark.parametrize("D,dtype", [(64, "fp16"), (64, "bf16"), (128, "fp16"), (128, "bf16")])
+def test_few_queries_masked_keys(D, dtype, Sq, masked, low, monkeypatch):
+    """The few-queries kernel: a wave's first tile, every wave's first tile, whole key splits, every key."""
+    from sageattention import sageattn
+
+    set_path(monkeypatch, direct=True)
+    q, k, v = inputs(1, 2, 1, Sq, 4096, D, dtype, low)
+    k[:, :, masked[0]:masked[1], 0] = lowest(dtype)
+    assert_close(sageattn(q, k, v, sm_scale=1.0, return_lse=True), exact(q, k, v, False), dtype)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_few_queries_masked_keys_int8(D, monkeypatch):
+    """INT8 scores overflow to -inf where the K scale is large enough (bf16 only)."""
+    from sageattention import sageattn
+
+    set_path(monkeypatch, direct=False)
+    q, k, v = inputs(1, 2, 1, 4, 4096, D, "bf16", False)
+    q[..., 0] = 20.0
+    want = sageattn(q, k[:, :, 64:], v[:, :, 64:], sm_scale=1.0, return_lse=True)
+    k[:, :, :64, 0] = lowest("bf16")
+    assert_close(sageattn(q, k, v, sm_scale=1.0, return_lse=True), want, "bf16")
