@@ -56,6 +56,7 @@
 //     merged by attn_merge_kernel with the partial LSEs.
 #include <algorithm>
 #include <atomic>
+#include <cfloat>
 #include <cmath>
 #include <type_traits>
 #include <utility>

@@ -90,3 +90,37 @@ def test_few_queries_masked_keys_int8(D, monkeypatch):
     want = sageattn(q, k[:, :, 64:], v[:, :, 64:], sm_scale=1.0, return_lse=True)
     k[:, :, :64, 0] = lowest("bf16")
     assert_close(sageattn(q, k, v, sm_scale=1.0, return_lse=True), want, "bf16")
+
+
+# block shapes of the general kernel: 128-row blocks in two key groups (17 key tiles), 128-row blocks (8), 256-row blocks,
+# causal 128-row blocks in two key groups
+SHAPES = [(3, 300, 1088, 64, False), (5, 600, 512, 64, False), (3, 300, 700, 128, False), (3, 500, 500, 64, True),
+          (3, 500, 500, 128, True)]
+
+
+@pytest.mark.parametrize("low", [False, True])
+@pytest.mark.parametrize("masked", [(0, 64), (64, 128), (0, 200)], ids=lambda m: f"keys{m[0]}-{m[1]}")
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("H,Sq,Sk,D,causal", SHAPES)
+def test_masked_keys(H, Sq, Sk, D, causal, dtype, masked, low, monkeypatch):
+    """The general kernel: the first key tile of the item, of its second key group, of both."""
+    from sageattention import sageattn
+
+    set_path(monkeypatch, direct=True)
+    q, k, v = inputs(1, H, H, Sq, Sk, D, dtype, low)
+    k[:, :, masked[0]:masked[1], 0] = lowest(dtype)
+    assert_close(sageattn(q, k, v, is_causal=causal, sm_scale=1.0, return_lse=True), exact(q, k, v, causal), dtype)
+
+
+@pytest.mark.parametrize("masked", [(0, 64), (64, 128)], ids=lambda m: f"keys{m[0]}-{m[1]}")
+@pytest.mark.parametrize("H,Sq,Sk,D", [(3, 300, 1088, 64), (5, 600, 512, 64), (3, 300, 700, 128)])
+def test_masked_keys_int8(H, Sq, Sk, D, masked, monkeypatch):
+    from sageattention import sageattn
+
+    set_path(monkeypatch, direct=False)
+    q, k, v = inputs(1, H, H, Sq, Sk, D, "bf16", False)
+    q[..., 0] = 20.0
+    live = [torch.cat([x[:, :, :masked[0]], x[:, :, masked[1]:]], 2) for x in (k, v)]
+    want = sageattn(q, *live, sm_scale=1.0, return_lse=True)
+    k[:, :, masked[0]:masked[1], 0] = lowest("bf16")
+    assert_close(sageattn(q, k, v, sm_scale=1.0, return_lse=True), want, "bf16")
