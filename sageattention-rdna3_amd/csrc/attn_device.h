@@ -98,6 +98,15 @@ __device__ __forceinline__ float xhalf_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Log-sum-exp of a row (natural log) from its reference max m and sum l in
+// log2 units: -inf without a live key (l = 0), NaN where the scores are.
+__device__ __forceinline__ float row_lse(float m, float l) {
+  return l == 0.0f ? -INFINITY : (m + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
+}
+
+// max(a, b) that keeps a NaN of either (fmaxf drops it)
+__device__ __forceinline__ float max_or_nan(float a, float b) { return (b > a || b != b) ? b : a; }
+
 // Uniform 64-bit pointer (the compiler cannot always prove it).
 template <typename T>
 __device__ __forceinline__ const T* uniform_ptr(const T* ptr) {

@@ -446,8 +446,9 @@ __global__ __launch_bounds__(kFewThreads, 1) void few_attn_kernel(FewParams p) {
       mw[w] = fast_exp2(mw[w] - mm);
       l = __builtin_fmaf(lw[w], mw[w], l);
     }
-    const float inv = (l > 0.0f) ? 1.0f / l : 0.0f;
-    const float lse = (l > 0.0f) ? (mm + __builtin_amdgcn_logf(l)) * 0.6931471805599453f : -INFINITY;
+    // no live key: output 0 and LSE -inf; a NaN sum (undefined scores) stays NaN in both
+    const float inv = (l == 0.0f) ? 0.0f : 1.0f / l;
+    const float lse = row_lse(mm, l);
     int g, tok;
     const bool ok = few_row(p, rg * RT + rt, m, g, tok);
     const int head = hk * p.group + g;
@@ -483,8 +484,9 @@ __global__ __launch_bounds__(kFewThreads, 1) void few_attn_kernel(FewParams p) {
   }
 }
 
-// Merge of the key splits (the formulas of attn_merge_kernel): D/4 lanes per
-// query row, which is one (b, query head, token); 8 splits' loads at a time.
+// Merge of the key splits (the formulas of attn_merge_kernel, a NaN LSE
+// included): D/4 lanes per query row, which is one (b, query head, token); 8
+// splits' loads at a time.
 template <int D, bool BF16>
 __global__ __launch_bounds__(256) void few_merge_kernel(FewParams p, int rt_rows, int64_t rows, FastDiv d_sq,
                                                         FastDiv d_hq, FastDiv d_group, FastDiv d_upt) {
@@ -507,10 +509,10 @@ __global__ __launch_bounds__(256) void few_merge_kernel(FewParams p, int rt_rows
   const float* lp = p.part_lse + base;
   const float* op = p.part + base * D + 4 * c;
   float mx = -INFINITY;
-  for (int s = 0; s < p.nsplit; ++s) mx = fmaxf(mx, lp[static_cast<int64_t>(s) * rt_rows]);
+  for (int s = 0; s < p.nsplit; ++s) mx = max_or_nan(mx, lp[static_cast<int64_t>(s) * rt_rows]);
   float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   float wsum = 0.0f;
-  if (mx > -INFINITY) {
+  if (mx != -INFINITY) {
     for (int s0 = 0; s0 < p.nsplit; s0 += 8) {
       float l[8];
       float4 v[8];
@@ -532,13 +534,13 @@ __global__ __launch_bounds__(256) void few_merge_kernel(FewParams p, int rt_rows
       }
     }
   }
-  const float inv = wsum > 0.0f ? 1.0f / wsum : 0.0f;
+  const float inv = wsum == 0.0f ? 0.0f : 1.0f / wsum;
   uint16_t* dst = static_cast<uint16_t*>(p.out) + static_cast<int64_t>(b) * p.o_sb + static_cast<int64_t>(head) * p.o_sh +
                   static_cast<int64_t>(tok) * p.o_sn + 4 * c;
   *reinterpret_cast<uint2*>(dst) =
       BF16 ? make_uint2(pack_bf16x2(acc.x * inv, acc.y * inv), pack_bf16x2(acc.z * inv, acc.w * inv))
            : make_uint2(pack_f16x2(acc.x * inv, acc.y * inv), pack_f16x2(acc.z * inv, acc.w * inv));
-  if (c == 0 && p.lse != nullptr) p.lse[row] = wsum > 0.0f ? mx + logf(wsum) : -INFINITY;
+  if (c == 0 && p.lse != nullptr) p.lse[row] = wsum == 0.0f ? -INFINITY : mx + logf(wsum);
 }
 
 // ---- host side

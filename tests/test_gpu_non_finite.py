@@ -1,6 +1,7 @@
 """Infinite and NaN scores through ``sageattn``: keys masked through a channel of K (-inf, or bf16's lowest value against
 a query entry of 2, whose product overflows in fp32).  A masked key has weight 0 wherever it lies: whole key tiles, the
-first tiles that a wave, a key group or a key split reads, whole splits, all keys (output 0, LSE -inf).
+first tiles that a wave, a key group or a key split reads, whole splits, all keys (output 0, LSE -inf).  A row whose scores
+are NaN gives a NaN output and a NaN LSE, with and without key splits.
 
 References: softmax attention in 64 bits over the same values (direct path), or the same call on the live keys alone
 (INT8 path; the masked ranges are whole scale groups, so the live keys quantise alike).  Tolerance: the parity tests'.
@@ -124,3 +125,44 @@ def test_masked_keys_int8(H, Sq, Sk, D, masked, monkeypatch):
     want = sageattn(q, *live, sm_scale=1.0, return_lse=True)
     k[:, :, masked[0]:masked[1], 0] = lowest("bf16")
     assert_close(sageattn(q, k, v, sm_scale=1.0, return_lse=True), want, "bf16")
+
+
+# (Hq, Hkv, Sq, Sk, D, causal, key splits): few queries with and without key splits, the general kernel unsplit and
+# split, causal
+NAN_CASES = [(4, 2, 3, 4096, 64, False, None), (4, 2, 3, 4096, 128, False, None), (4, 2, 3, 90, 128, False, None),
+             (4, 2, 3, 90, 64, False, None), (4, 2, 300, 1088, 64, False, 1), (4, 2, 300, 1088, 64, False, 3),
+             (4, 2, 300, 700, 128, False, 1), (4, 2, 300, 700, 128, False, 3), (4, 2, 300, 300, 128, True, None),
+             (4, 2, 300, 300, 64, True, None)]
+NAN_IDS = [f"H{c[0]}q{c[2]}kv{c[3]}D{c[4]}{'_c' if c[5] else ''}_s{c[6]}" for c in NAN_CASES]
+
+
+@pytest.mark.parametrize("direct", [True, False])
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("Hq,Hkv,Sq,Sk,D,causal,splits", NAN_CASES, ids=NAN_IDS)
+def test_nan_query(Hq, Hkv, Sq, Sk, D, causal, splits, dtype, direct, monkeypatch):
+    """A query without a defined result stays visible: NaN output and NaN LSE, never the zeros of a row without keys.
+    Direct: one NaN in the query.  INT8: an infinite entry (infinite scale of its 32-token group: 0 * inf scores)."""
+    from sageattention import sageattn
+
+    set_path(monkeypatch, direct, splits)
+    q, k, v = inputs(1, Hq, Hkv, Sq, Sk, D, dtype, False)
+    o, lse = (x.clone() for x in sageattn(q, k, v, is_causal=causal, sm_scale=0.3, return_lse=True))
+    q[0, 1, 1, 5] = float("nan") if direct else float("inf")
+    rows = slice(1, 2) if direct else slice(0, min(Sq, 32))
+    o[0, 1, rows], lse[0, 1, rows] = float("nan"), float("nan")
+    assert_close(sageattn(q, k, v, is_causal=causal, sm_scale=0.3, return_lse=True), (o, lse), dtype)
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("Hq,Hkv,Sq,Sk,D,causal,splits", NAN_CASES, ids=NAN_IDS)
+def test_nan_key(Hq, Hkv, Sq, Sk, D, causal, splits, dtype, monkeypatch):
+    """A NaN in one key of the direct path reaches the output and the LSE of every row that reads the key."""
+    from sageattention import sageattn
+
+    set_path(monkeypatch, True, splits)
+    q, k, v = inputs(1, Hq, Hkv, Sq, Sk, D, dtype, False)
+    o, lse = (x.clone() for x in sageattn(q, k, v, is_causal=causal, sm_scale=0.3, return_lse=True))
+    k[0, 1, 70, 5] = float("nan")
+    first = 70 if causal else 0
+    o[0, Hq // 2:, first:], lse[0, Hq // 2:, first:] = float("nan"), float("nan")
+    assert_close(sageattn(q, k, v, is_causal=causal, sm_scale=0.3, return_lse=True), (o, lse), dtype)
