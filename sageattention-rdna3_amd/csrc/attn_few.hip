@@ -346,18 +346,28 @@ __global__ __launch_bounds__(kFewThreads, 1) void few_attn_kernel(FewParams p) {
     half8_t pf[RT][2];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-      float y[16];
-      float mx = -INFINITY;
       const float sc[2] = {qs[rt] * ks[0], qs[rt] * ks[1]};
+      float y[16];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) y[r] = static_cast<float>(s[rt][r]) * sc[r >> 3];
-      if (ragged) {
+      for (int r = 0; r < 16; ++r) y[r] = static_cast<float>(s[rt][r]);
+      auto mask = [&]() __attribute__((always_inline)) {
+        if (ragged) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (key0 + 16 * (r >> 3) + 8 * hh + (r & 7) >= p.sk) y[r] = -INFINITY;
+          for (int r = 0; r < 16; ++r)
+            if (key0 + 16 * (r >> 3) + 8 * hh + (r & 7) >= p.sk) y[r] = -INFINITY;
+        }
+      };
+      mask();
+      // the row's largest score: each key group's largest accumulator, scaled (scales are not negative; fmaxf
+      // drops the NaN that a scale of 0 makes of a group without a live key)
+      float mx = -INFINITY;
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        float gm = y[8 * g];
+#pragma unroll
+        for (int r = 1; r < 8; ++r) gm = __builtin_fmaxf(gm, y[8 * g + r]);
+        mx = __builtin_fmaxf(mx, gm * sc[g]);
       }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) mx = __builtin_fmaxf(mx, y[r]);
       mx = xhalf_max(mx);
       // lazy reference max, as in attn_body.inc: it moves when a row's tile max
       // passes it by more than kFewRescale, so p stays below 2^8.  It starts at
@@ -377,11 +387,15 @@ __global__ __launch_bounds__(kFewThreads, 1) void few_attn_kernel(FewParams p) {
           for (int r = 0; r < 16; ++r) o[rt][db][r] *= alpha;
         }
       }
+      // score - max in one rounding: scores may be far larger than their differences
+#pragma unroll
+      for (int r = 0; r < 16; ++r) y[r] = __builtin_fmaf(y[r], sc[r >> 3], -m_run[rt]);
+      mask();
       float sum[2] = {0.0f, 0.0f};
       uint32_t pw[8];
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
-        const float e0 = fast_exp2(y[r] - m_run[rt]), e1 = fast_exp2(y[r + 1] - m_run[rt]);
+        const float e0 = fast_exp2(y[r]), e1 = fast_exp2(y[r + 1]);
         sum[0] += e0;
         sum[1] += e1;
         pw[r / 2] = pack_f16x2(e0, e1);
