@@ -109,25 +109,63 @@ constexpr int64_t kVRowsMaxQueriesCausal = 8192;
 // Few query rows per kv head against the key range: one pass over K and V in
 // place for the rows of all its query heads (sage_attn_few_fwd).  The general
 // path quantises K and transposes V first (INT8), pads each query head to 128
-// or 256 rows and reads K/V once per query head.  The rows are packed into
-// 32-row tiles; a launch of many tiles re-reads K/V per two of them.  Whole
-// call on MI355X, general / few: INT8, one tile: B8 Hq32 Hkv8 Sq1 Sk8192 D128
-// 225 / 55 us, B4 Hq32 Hkv4 Sq8 Sk16384 204 / 46; 4 tiles: B4 H16 Sq128 Sk4096
-// 66 / 39, H8 Sk8192 D64 26.6 / 23.9; 8 tiles: B1 H8 Sq256 Sk8192 D128 42 / 36,
-// D64 29.2 / 25.4; 16 tiles: 46 / 53, 32 / 34.  Direct: one tile B8 H8 Sq2
-// Sk4096 D64 34 / 17; 3 tiles H16 Sk2048 D128 19.5 / 18.5, H16 Sk1024 D64 12.4 /
-// 12.0; 4 tiles of 128-row heads 20.4 / 22.1; 8 tiles of 40-row heads (B2 Hq32
-// Hkv8 Sk3000) 39 / 22.
+// or 256 rows and reads K/V once per query head.  The few-queries kernel packs
+// the rows into 32-row tiles, two of them a block ("row group"), and runs one
+// 4-wave block per CU (its rings fill the LDS), where the general kernel hosts
+// two 128-row blocks a CU at D = 64; every row group reads K/V again (INT8:
+// and quantises K again).  Whole call on MI355X, general / few in us, D64 fp16,
+// D128 bf16, H the (kv) heads of all batches; the lines below were drawn over
+// 4700 shapes of 4 to 1024 kv heads, 1 to 8 query heads each, 1 to 256 queries
+// and 32 to 16384 keys.
 constexpr int64_t kFewMaxTiles = 8;
 constexpr int64_t kFewMaxTilesDirect = 3;   // direct path, heads of more than kFewShortHead rows
 constexpr int64_t kFewShortHead = 64;
+constexpr int64_t kCus = 256;               // MI355X
+
+bool few_pays(int64_t b, int64_t hq, int64_t hkv, int64_t sq, int64_t sk, int64_t d, bool direct) {
+  if (sq <= 0 || sk <= 0 || sq > 32 * kFewMaxTiles) return false;
+  const int64_t group = hq / hkv;
+  const int64_t units = group * ((sq + 31) / 32);  // 32-token groups of the heads, never cut by a tile
+  const int64_t per_tile = 32 / std::min<int64_t>(sq, 32);
+  const int64_t tiles = (units + per_tile - 1) / per_tile;
+  if (tiles > (direct && sq > kFewShortHead ? kFewMaxTilesDirect : kFewMaxTiles)) return false;
+  // blocks of either kernel and the rounds over the CUs they take (before key splits)
+  const int64_t row_groups = tiles > 1 ? (tiles + 1) / 2 : 1;
+  const int64_t rows = d == 64 ? 128 : 256, per_cu = d == 64 ? 2 : 1;
+  const int64_t q_blocks = group * ((sq + rows - 1) / rows);
+  const int64_t few_blocks = b * hkv * row_groups, gen_blocks = b * hkv * q_blocks;
+  const int64_t few_rounds = (few_blocks + kCus - 1) / kCus;
+  const int64_t gen_rounds = (gen_blocks + per_cu * kCus - 1) / (per_cu * kCus);
+  if (direct) {
+    // more rounds than the general kernel: H1024 Sq64 Sk64 D64 12.0 / 22.2, Sq96 Sk64 12.8 / 42.0, Sq1 Sk1024 50.5 /
+    // 55.0; Sq96 Sk64 D128 31.0 / 65.4.  As many or fewer: H256 Sq1 Sk256 D64 8.5 / 6.6; Hq128 Hkv32 Sq1 Sk1024 D128
+    // 29.8 / 11.6
+    if (few_rounds > gen_rounds) return false;
+    // several row tiles against one key tile of the general kernel (two where the launch has several rounds): half of
+    // a block's waves have no key tile.  H64 Sq64 Sk64 D64 5.4 / 6.1, D128 7.9 / 9.0; Sk256 D128 13.0 / 10.9
+    if (tiles > 1 && few_rounds == gen_rounds && sk <= (few_rounds > 1 ? 128 : 64)) return false;
+    // few ungrouped heads and long keys: the general kernel's key splits fill the CUs as well, and merge faster.  H8
+    // Sq1 Sk4096 D64 11.5 / 14.2, Sq64 Sk1024 10.3 / 11.2; H64 Sq64 Sk1024 15.8 / 14.1; H8 Sq64 Sk4096 D128 18.3 / 22.2
+    if (group == 1 && gen_blocks <= (d == 64 ? 32 : 8) &&
+        sk > (d == 64 ? (tiles > 1 ? 1000 : 2000) : (tiles > 1 ? 3000 : sk)))
+      return false;
+  } else {
+    // K quantised by each of 4 row groups, and more rounds: H128 Sq256 Sk2048 D128 89 / 102; Hq1024 Hkv256 Sq64 Sk512
+    // D64 36 / 51.  Two row groups: from 4 times the rounds, H512 Sq128 Sk512 D64 34 / 57, H256 Sk2048 D128 125 / 100
+    if (row_groups > 2 && few_rounds > gen_rounds) return false;
+    if (row_groups == 2 && few_rounds >= 4 * gen_rounds) return false;
+    // ... in one round, where the general kernel reads K/V half as often and the keys are long: H64 Sq256 Sk8192 D128
+    // 146 / 184, Sk2048 60 / 55
+    if (row_groups > 2 && row_groups >= 2 * q_blocks && sk >= 4096 && 2 * few_blocks >= kCus) return false;
+    // little K and V and few query heads in all: the merge of up to 32 key splits outweighs the quantisation pass.  H4
+    // Sq1 Sk8192 D64 20.7 / 23.7, Sq128 22.4 / 29.5; H4 Sq1 Sk5000 19.0 / 16.2, Hq64 Hkv8 Sq1 Sk8192 33.2 / 24.7
+    if (d == 64 && sk > 6144 && few_blocks * sk <= 65536 && gen_blocks <= 16) return false;
+  }
+  return true;
+}
 
 bool few_queries(const Dims& q, const Dims& k, const Dims& v, bool direct) {
-  if (q.n <= 0 || k.n <= 0 || q.n > 32 * kFewMaxTiles) return false;
-  const int64_t units = q.h / k.h * ((q.n + 31) / 32);  // 32-token groups of the heads, never cut by a tile
-  const int64_t per_tile = 32 / std::min<int64_t>(q.n, 32);
-  const int64_t tiles = (units + per_tile - 1) / per_tile;
-  if (tiles > (direct && q.n > kFewShortHead ? kFewMaxTilesDirect : kFewMaxTiles)) return false;
+  if (!few_pays(q.b, q.h, k.h, q.n, k.n, q.d, direct)) return false;
   constexpr int64_t kPastEnd = 24 * 32;  // keys past the last that the kernel's loads address (they read as zero)
   return k.sn >= q.d && v.sn >= q.d && (k.n + kPastEnd) * k.sn * 2 <= UINT32_MAX &&
          (k.n + kPastEnd) * v.sn * 2 <= UINT32_MAX && q.b * q.h <= INT32_MAX / SAGE_FEW_MAX_ROWS;
@@ -324,6 +362,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("num_splits"), py::arg("stream"));
   m.def("sageattn_plain", &sageattn_plain, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("hnd"),
         py::arg("is_causal"), py::arg("sm_scale"), py::arg("return_lse"), py::arg("smooth_k"), py::arg("stream"));
+  m.def("few_pays", &few_pays, py::arg("batch"), py::arg("q_heads"), py::arg("kv_heads"), py::arg("q_len"),
+        py::arg("kv_len"), py::arg("head_dim"), py::arg("direct"));
   m.def("default_direct", &default_direct, py::arg("head_dim"), py::arg("q_len"), py::arg("kv_len"),
         py::arg("is_causal"), py::arg("hnd"));
   py::register_exception_translator([](std::exception_ptr p) {

@@ -98,3 +98,32 @@ def test_few_queries_graph_capture_and_replay(force_i8, monkeypatch):
         torch.cuda.synchronize()
         assert torch.equal(out, ref)
         assert torch.equal(sageattn(q, k, v), ref)
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk,D,dtype,direct", [
+    (2, 2, 64, 1500, 64, torch.float16, True),     # few heads, long keys, two row tiles
+    (1, 1, 1, 20011, 64, torch.bfloat16, False),   # little K and V in all: many key splits
+    (20, 16, 96, 64, 64, torch.bfloat16, True),    # a batch of windows: more blocks than CUs, waves without a tile
+    (20, 16, 49, 49, 128, torch.float16, True),
+])
+def test_few_queries_entry_where_the_general_kernel_is_faster(B, H, Sq, Sk, D, dtype, direct, monkeypatch):
+    """Shapes that ``sageattn`` leaves to the general kernel, through the C entry, against ``sageattn``: both round P and
+    the output, so 2^-9 + 2^-10 (bf16: 2^-7) of the value each."""
+    from sageattention import _capi, ops, sageattn
+
+    for name in ("D64", "D64_CROSS", "D128", "D128_CROSS"):
+        monkeypatch.setenv("SAGEATTN_DIRECT_THRESHOLD_" + name, "100000" if direct else "-1")
+    monkeypatch.delenv("SAGEATTN_KV_SPLITS", raising=False)
+    g = torch.Generator().manual_seed(Sk)
+    q, k, v = (torch.randn(B, H, s, D, generator=g).to(dtype).cuda() for s in (Sq, Sk, Sk))
+    w, wl = sageattn(q, k, v, return_lse=True)
+    o, lse = torch.full_like(q, float("nan")), torch.full_like(wl, float("nan"))
+    ws_bytes = _capi.query("sage_attn_few_workspace_bytes", B, H, H, Sq, Sk, D)
+    ws = torch.empty(max(ws_bytes, 16), device="cuda", dtype=torch.uint8)
+    strides = [x.stride(i) for x in (q, k, v, o) for i in range(3)]
+    _capi.call("sage_attn_few_fwd", 0 if direct else 1, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+               lse.data_ptr(), 1 if dtype == torch.bfloat16 else 0, B, H, H, Sq, Sk, D, *strides, D ** -0.5,
+               ws.data_ptr() if ws_bytes else None, ws_bytes, ops._stream(q))
+    rtol = 1.6e-2 if dtype == torch.bfloat16 else 4e-3
+    assert torch.allclose(o.float(), w.float(), atol=2e-3, rtol=rtol)
+    assert torch.allclose(lse, wl, rtol=2e-6, atol=2e-4)
