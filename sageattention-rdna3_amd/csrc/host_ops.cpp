@@ -171,6 +171,24 @@ bool few_queries(const Dims& q, const Dims& k, const Dims& v, bool direct) {
          (k.n + kPastEnd) * v.sn * 2 <= UINT32_MAX && q.b * q.h <= INT32_MAX / SAGE_FEW_MAX_ROWS;
 }
 
+// Direct path, bf16 inputs: whether the kernel reads V in place.  Every block
+// then converts its V tiles to fp16, about 24 (D = 64) or 30 (D = 128) ns per
+// million query-key pairs of the launch; the V_T pass saved is a launch and
+// twice V's bytes, about 1.9 us + 0.35 us per MB of V.  Fitted to 630 shapes of
+// 256 to 8192 queries and 77 to 6144 keys (the side taken is at most 3%
+// slower).  Whole call on MI355X, V_T / in place in us: D128 H16 Sq4096 Sk512
+// 27.9 / 25.0, causal H32 S2048 58.4 / 52.0; D64 H20 S1024 17.2 / 14.7, causal
+// H32 S4096 90.7 / 83.1; H32 Sq5529 Sk6144 296 / 315, Hq32 Hkv8 290 / 312,
+// causal S5000 210 / 217, B2 Hq32 Hkv4 Sq8192 Sk2048 298 / 323.  (fp16 needs no
+// conversion and is at most 1.5% slower in place.)
+bool bf16_v_in_place(int64_t b, int64_t hq, int64_t hkv, int64_t sq, int64_t sk, int64_t d, bool causal) {
+  const double n = static_cast<double>(std::min(sq, sk)), rows = static_cast<double>(sq), keys = static_cast<double>(sk);
+  const double pairs = causal ? n * (n + 1) / 2 + (rows - n) * keys : rows * keys;  // of a head
+  const double convert_us = static_cast<double>(b * hq) * pairs * (d == 64 ? 24e-9 : 30e-9);
+  const double pass_us = 1.9 + 0.35e-6 * static_cast<double>(b * hkv * sk * d * 2);
+  return convert_us < pass_us;
+}
+
 py::object sageattn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, int64_t layout, bool is_causal, double sm_scale,
                         bool return_lse, bool smooth_k, bool direct, int64_t num_splits, int64_t stream_handle) {
   if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4) throw py::value_error("q, k and v must be 4-D tensors");
@@ -219,11 +237,11 @@ py::object sageattn_fwd(at::Tensor q, at::Tensor k, at::Tensor v, int64_t layout
     int64_t ws_bytes = 0;
     at::Tensor ws = split_workspace(false, qd, Sk, is_causal, num_splits, q, &ws_bytes);
     // V read in place: one launch, the same output bit for bit as the V_T path (kept for V rows that overlap or
-    // span more than 32-bit offsets).  Whole call on MI355X, V_T / in place: fp16 D64 causal B1 H32 S2048 37.5 / 29.8
-    // us, H20 S3072 50.4 / 43.6, H16 S6144 142 / 133; D64 non-causal B1 H20 S1536 23.9 / 19.8, S2304 43.8 / 39.8;
-    // bf16 D128 B1 H16 Sq4096 kv512 27.9 / 25.0, kv154 19.9 / 16.6, causal H32 S2048 58.4 / 52.0, H8 S1024 22.4 /
-    // 21.6, B2 H32 S2048 152 / 150; bf16 D64 H20 S1024 17.2 / 14.7, causal H16 S6144 147.8 / 143.3
-    const bool v_rows = vd.sn >= D && (Sk + 5 * SAGE_VT_ALIGN) * vd.sn * 2 <= UINT32_MAX;
+    // span more than 32-bit offsets, and for bf16 where the conversion costs more).  Whole call on MI355X, V_T / in
+    // place: fp16 D64 causal B1 H32 S2048 37.5 / 29.8 us, H20 S3072 50.4 / 43.6, H16 S6144 142 / 133; D64 non-causal B1
+    // H20 S1536 23.9 / 19.8, S2304 43.8 / 39.8
+    const bool v_rows = vd.sn >= D && (Sk + 5 * SAGE_VT_ALIGN) * vd.sn * 2 <= UINT32_MAX &&
+                        (dtype == SAGE_DTYPE_F16 || bf16_v_in_place(B, Hq, Hkv, Sq, Sk, D, is_causal));
     if (v_rows && dtype == SAGE_DTYPE_BF16) {
       check("sage_attn_direct_fwd_vrows_bf16",
             sage_attn_direct_fwd_vrows_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
@@ -364,6 +382,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("is_causal"), py::arg("sm_scale"), py::arg("return_lse"), py::arg("smooth_k"), py::arg("stream"));
   m.def("few_pays", &few_pays, py::arg("batch"), py::arg("q_heads"), py::arg("kv_heads"), py::arg("q_len"),
         py::arg("kv_len"), py::arg("head_dim"), py::arg("direct"));
+  m.def("bf16_v_in_place", &bf16_v_in_place, py::arg("batch"), py::arg("q_heads"), py::arg("kv_heads"), py::arg("q_len"),
+        py::arg("kv_len"), py::arg("head_dim"), py::arg("is_causal"));
   m.def("default_direct", &default_direct, py::arg("head_dim"), py::arg("q_len"), py::arg("kv_len"),
         py::arg("is_causal"), py::arg("hnd"));
   py::register_exception_translator([](std::exception_ptr p) {

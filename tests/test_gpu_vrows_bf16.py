@@ -62,3 +62,26 @@ def test_bf16_v_in_place_equals_vt_path(cfg, splits):
     assert torch.equal(torch.isnan(o), torch.isnan(o_ref))
     assert torch.equal(torch.nan_to_num(o.float()), torch.nan_to_num(o_ref.float()))
     assert torch.equal(lse, lse_ref)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_sageattn_across_the_in_place_line(causal, monkeypatch):
+    """``sageattn`` on a launch that takes the V_T pass against the entry that reads V in place: the same bits."""
+    from sageattention import _capi, core, ops, sageattn
+
+    for name in ("D64", "D64_CAUSAL", "D64_CROSS"):
+        monkeypatch.delenv("SAGEATTN_DIRECT_THRESHOLD_" + name, raising=False)
+    monkeypatch.delenv("SAGEATTN_KV_SPLITS", raising=False)
+    B, Hq, Hkv, Sq, Sk, D = (1, 16, 1, 4001 if causal else 2700, 4001 if causal else 3000, 64)
+    assert not core._host().bf16_v_in_place(B, Hq, Hkv, Sq, Sk, D, causal)
+    g = torch.Generator().manual_seed(7)
+    q, k, v = (torch.randn(B, h, s, D, generator=g).bfloat16().cuda() for h, s in ((Hq, Sq), (Hkv, Sk), (Hkv, Sk)))
+    ref, lse_ref = sageattn(q, k, v, is_causal=causal, return_lse=True)
+    o, lse = torch.full_like(q, float("nan")), torch.full_like(lse_ref, float("nan"))
+    ws_bytes = 0 if causal else _capi.query("sage_attn_workspace_bytes", 0, B, Hq, Sq, Sk, D, 0, 0)
+    ws = torch.empty(max(ws_bytes, 16), device="cuda", dtype=torch.uint8)
+    strides = [x.stride(i) for x in (q, k, v, o) for i in range(3)]
+    _capi.call("sage_attn_direct_fwd_vrows_bf16", q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
+               B, Hq, Hkv, Sq, Sk, D, *strides, int(causal), D ** -0.5, 0, ws.data_ptr() if ws_bytes else None, ws_bytes,
+               ops._stream(q))
+    assert torch.equal(o, ref) and torch.equal(lse, lse_ref)

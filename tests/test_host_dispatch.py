@@ -1,5 +1,6 @@
 """The compiled host layer's dispatch: its direct / INT8 choice (default thresholds) equals core.use_direct_path over both
-head dims, layouts, causality and lengths around every threshold; which calls take the few-queries kernel."""
+head dims, layouts, causality and lengths around every threshold; which calls take the few-queries kernel
+and which bf16 ones read V in place."""
 import itertools
 
 
@@ -50,3 +51,18 @@ def test_few_queries_rule():
         assert few(*args), args
     for args in general:
         assert not few(*args), args
+
+
+def test_bf16_v_in_place_rule():
+    """Direct path, bf16: V in place on short and causal launches, through the V_T pass where the conversion of the V
+    tiles by every query block costs more than the pass."""
+    from sageattention import core
+
+    rule = core._host().bf16_v_in_place
+    for args in [(1, 16, 16, 4096, 512, 128, False), (1, 32, 32, 2048, 2048, 128, True), (1, 20, 20, 1024, 1024, 64, False),
+                 (1, 32, 32, 4096, 4096, 64, True), (1, 1, 1, 1, 1, 64, False), (1, 10, 10, 4096, 77, 64, False),
+                 (1, 4, 4, 100, 6144, 64, True), (1, 4, 4, 100, 0, 64, False)]:
+        assert rule(*args), args
+    for args in [(1, 32, 32, 5529, 6144, 64, False), (1, 32, 8, 5529, 6144, 64, False), (1, 32, 8, 5000, 5000, 64, True),
+                 (2, 32, 4, 8192, 2048, 64, False), (2, 32, 4, 8192, 2048, 128, False)]:
+        assert not rule(*args), args
