@@ -104,9 +104,6 @@ __device__ __forceinline__ float row_lse(float m, float l) {
   return l == 0.0f ? -INFINITY : (m + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
 }
 
-// max(a, b) that keeps a NaN of either (fmaxf drops it)
-__device__ __forceinline__ float max_or_nan(float a, float b) { return (b > a || b != b) ? b : a; }
-
 // Uniform 64-bit pointer (the compiler cannot always prove it).
 template <typename T>
 __device__ __forceinline__ const T* uniform_ptr(const T* ptr) {

@@ -523,29 +523,28 @@ __global__ __launch_bounds__(256) void few_merge_kernel(FewParams p, int rt_rows
   const float* lp = p.part_lse + base;
   const float* op = p.part + base * D + 4 * c;
   float mx = -INFINITY;
-  for (int s = 0; s < p.nsplit; ++s) mx = max_or_nan(mx, lp[static_cast<int64_t>(s) * rt_rows]);
+  for (int s = 0; s < p.nsplit; ++s) mx = fmaxf(mx, lp[static_cast<int64_t>(s) * rt_rows]);
   float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   float wsum = 0.0f;
-  if (mx != -INFINITY) {
-    for (int s0 = 0; s0 < p.nsplit; s0 += 8) {
-      float l[8];
-      float4 v[8];
+  if (mx == -INFINITY) mx = 0.0f;  // no live key, or only NaN ones: weights 0 or NaN
+  for (int s0 = 0; s0 < p.nsplit; s0 += 8) {
+    float l[8];
+    float4 v[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int64_t s = min(s0 + i, p.nsplit - 1);
-        l[i] = s0 + i < p.nsplit ? lp[s * rt_rows] : -INFINITY;
-        v[i] = *reinterpret_cast<const float4*>(op + s * rt_rows * D);
-      }
+    for (int i = 0; i < 8; ++i) {
+      const int64_t s = min(s0 + i, p.nsplit - 1);
+      l[i] = s0 + i < p.nsplit ? lp[s * rt_rows] : -INFINITY;
+      v[i] = *reinterpret_cast<const float4*>(op + s * rt_rows * D);
+    }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if (s0 + i >= p.nsplit) break;
-        const float w = expf(l[i] - mx);
-        wsum += w;
-        acc.x += w * v[i].x;
-        acc.y += w * v[i].y;
-        acc.z += w * v[i].z;
-        acc.w += w * v[i].w;
-      }
+    for (int i = 0; i < 8; ++i) {
+      if (s0 + i >= p.nsplit) break;
+      const float w = expf(l[i] - mx);
+      wsum += w;
+      acc.x += w * v[i].x;
+      acc.y += w * v[i].y;
+      acc.z += w * v[i].z;
+      acc.w += w * v[i].w;
     }
   }
   const float inv = wsum == 0.0f ? 0.0f : 1.0f / wsum;
