@@ -161,7 +161,7 @@ int sage_attn_i8_fwd(const int8_t* q_i8, const int8_t* k_i8, const void* value_t
  * contiguous (4-byte aligned; NULL = not written) receives
  * ln(sum_j exp(s_ij)) over the natural-log scores s_ij = q_i.k_j * sm_scale
  * after dequantisation (the log2-domain score times ln 2), -inf for a row with
- * no live key.  The reference's return_lse returns a zero placeholder instead
+ * no live key (output 0), NaN where the output is NaN.  The reference's return_lse returns a zero placeholder instead
  * (sageattention/core.py:203-211); this is the value that placeholder stands
  * for, usable to merge partial attentions over split key ranges.
  */
@@ -179,9 +179,10 @@ int sage_attn_i8_fwd_lse(const int8_t* q_i8, const int8_t* k_i8, const void* val
  * q-blocks would fill at most half the CUs, and for causal launches whose
  * 256-row q-blocks fill at most one round when a cost model of the schedule
  * rates 128-row q-blocks faster; R = 256 otherwise (one block per CU).
- * Non-causal 128-row blocks run two per CU, causal ones one per CU (more of
- * them than CUs run as a persistent grid, a heavy and a light q-block per
- * block); for a non-causal
+ * Non-causal 128-row blocks run two per CU, or one per CU in two key groups
+ * where the launch has at most one item per CU and at least 16 key tiles an
+ * item; causal ones one per CU in two key groups (more of them than CUs run as
+ * a persistent grid, a heavy and a light q-block per block).  For a non-causal
  * launch that leaves compute units idle
  * (fewer blocks than CUs, or a last round partly filled) the key range of
  * some or all blocks can be split into parts whose fp32 partial outputs and

@@ -84,11 +84,12 @@ namespace sage {
 // kernel at B1 H20 S1024: 21.3 -> 15.6 us; INT8 at B1 H10 S4096: 65.9 -> 56.2
 // us); causal launches of one or more full rounds +2% to +6% and D = 128
 // non-causal launches with key splits +3% to +4% (the doubled tile traffic),
-// so those stay on w8.  g2 against w4, whole sageattn, same box: INT8 causal
-// B1 H8 S4096 D128 64.8 -> 61.3 us, H4 S8192 107 -> 98; direct causal B1 H16
-// S2048 D128 46.3 -> 37.9, H8 S1024 D128 23.8 -> 22.4, H16 S2048 D64 29.2 ->
-// 27.1, H8 S7000 D64 (INT8) 77.3 -> 69.8, H32 S2048 D64 39.7 -> 38.6; paired
-// causal D128 within 1%; direct non-causal B1 H20 S1024 D64 19.7 -> 16.6.
+// so those stay on w8.  w4 / g2, whole sageattn, bf16, same box (causal w4 in a
+// build that has those kernels): INT8 causal B1 H8 S4096 D128 65.1 / 60.9 us,
+// H4 S8192 107.8 / 97.4, D64 H8 S6144 68.0 / 59.4; direct causal B1 H16 S2048
+// D128 40.7 / 37.6, H8 S1024 24.1 / 22.8, D64 H16 S2048 27.8 / 24.5; paired
+// causal: direct H32 S2048 D128 54.0 / 52.9, D64 33.7 / 30.8, INT8 H16 S4096
+// D128 82.0 / 80.9; non-causal as at kMinGroupTiles below.
 // The stamps build (build.py --stamps, SAGE_STAMPS=1) adds per-wave cycle
 // stamps to the attention kernels (attn_body.inc, StampField) and the two
 // functions below that read them; the default build has neither.
@@ -129,29 +130,30 @@ constexpr bool kSmallShape = true;
 }  // namespace g2
 
 // A lone 128-row block on a CU takes this fraction of a 256-row block's time
-// per key tile step (MI355X, B1 H32 S2048 causal: the D = 128 direct kernel
-// 0.97 against 1.38 us; fitted to the Q-fused INT8 kernel's paired launches at
-// B1 H16 S4096 and B1 H32 S2048: 0.77).
+// per key tile step.  Fitted to 4-wave blocks (MI355X, B1 H32 S2048 causal: the
+// D = 128 direct kernel 0.97 against 1.38 us; the Q-fused INT8 kernel's paired
+// launches at B1 H16 S4096 and B1 H32 S2048: 0.77).  The g2 blocks that run
+// instead are 1-17% faster, so a launch taken by these factors gains, and a few
+// that would gain are left in w8 (below).
 constexpr double kLoneHalfBlockTileDirect = 0.70;
 constexpr double kLoneHalfBlockTileI8 = 0.77;
 
 // Whether a launch runs 128-row q-blocks (in w4 or g2, by key_groups): D = 64
-// non-causal launches, and causal ones.  The causal timings below compare the
-// 256-row blocks with 4-wave 128-row ones; g2 is faster still.  128 rows for causal
-// launches whose 256-row q-blocks would fill at most half the CUs (their
-// 128-row q-blocks then fill twice as many, one block per CU; B1 H8 S4096
-// D128 INT8: -27%; the D = 128 direct kernel, whose 98 KB of LDS fits once per
-// CU, at B1 H8/H16 S1024-2048: -27% to -32%); w8 for the rest (a causal launch
-// of 2048 +4% in 128 rows).  A causal launch also runs 128 rows when its 256-row
-// q-blocks fill one round and the causal cost model rates the 128-row q-blocks
-// faster: with one block resident per CU they run as a persistent grid in
-// which the snake schedule gives each block a heavy and a light q-block.
-// D = 128 direct kernel: B1 H32 S2048, B2 H16 S2048 -17%, B1 H24 S2048 -15%,
-// B1 H16 S4096 -21%; Q-fused INT8 kernel: B1 H16 S4096, B2 H8 S4096 -15%,
-// B1 H12 S4096 -19%, B1 H32 S2048 -10%; D = 64: direct B1 H32 S2048 -16%,
-// B1 H20 S3072 -5%, INT8 B1 H16 S4096 -16%, B1 H32 S2048 -9%.  The model
-// keeps B1 H32 S1536 D128 direct in w8, where a block would get two heavy
-// q-blocks (+15% in w4).
+// non-causal launches, and causal ones.  128 rows for causal launches whose
+// 256-row q-blocks would fill at most half the CUs (their 128-row q-blocks then
+// fill twice as many, one block per CU); w8 for launches of more than a round.
+// A causal launch also runs 128 rows when its 256-row q-blocks fill at most one
+// round and the causal cost model rates the 128-row q-blocks faster: with one
+// block resident per CU they run as a persistent grid in which the snake
+// schedule gives each block a heavy and a light q-block.  (The model walks w4's
+// schedule, which is g2's: both have 128 rows and, causal, one block per CU.)
+// Whole sageattn, w8 / 128 rows as g2, causal, B1, bf16, same box: half a round
+// INT8 H8 S4096 D128 91.1 / 60.9 us, direct H8 S1024 D128 31.5 / 22.8, H16 S2048
+// 54.0 / 37.6; one round direct D128 H32 S2048 59.5 / 52.9, H24 54.0 / 45.6, D64
+// H32 S2048 38.7 / 30.8, H20 S3072 52.8 / 46.5, INT8 H16 S4096 D128 97.8 / 80.9,
+// D64 72.0 / 55.9, H12 S4096 D128 92.4 / 74.4.  The model rightly keeps H32 S1536
+// D128 direct in w8 (46.0 / 53.7: a block would get two heavy q-blocks), and
+// INT8 S3072 wrongly (H12-H20 D64 57.9 / 51.2, D128 76.0 / 72.2).
 bool small_blocks(int64_t head_dim, int is_causal, int64_t batch, int64_t q_heads, int64_t q_len, int64_t kv_len,
                   bool direct) {
   if (is_causal == 0) return head_dim == 64;
@@ -172,9 +174,13 @@ bool small_blocks(int64_t head_dim, int is_causal, int64_t batch, int64_t q_head
 // whose items (q-blocks, or key pieces of split ones) fit one per CU and have
 // at least this many key tiles.  With more items than CUs w4 hosts two blocks
 // a CU, which share no barrier (B1 H10 S4096 D64, 512 items: w4 60 us, g2 65);
-// with fewer tiles the merge and the doubled prologue outweigh the halved
-// steps (kernel alone, w4 / g2: 4 tiles 8.0 / 8.8 us, 8 tiles 10.6 / 10.9, 12
-// tiles 12.8 / 13.2, 16 tiles 19.7 / 16.9, 36 tiles whole call 31.8 / 29.6).
+// with few tiles the merge and the doubled prologue outweigh the halved steps.
+// Whole call, w4 / g2, B1 H20 Sq1024 D64 (160 items; 80 to 240 items alike):
+// direct fp16 4 tiles 7.9 / 8.7 us, 8 10.2 / 10.7, 12 12.5 / 12.5, 14 13.8 /
+// 13.4, 16 14.9 / 14.4, 24 19.6 / 18.1, 32 24.1 / 21.8; bf16 16 15.9 / 15.0;
+// INT8 fp16 8 17.3 / 17.4, 16 22.1 / 21.2, 48 41.3 / 36.2.  Even at 12; from 16
+// on g2 gains in every kind.  Per piece of split items the same: H10, 2 or 3
+// pieces of 10 tiles 17.4 / 18.3, 3 of 16 29.3 / 28.9 (INT8).
 constexpr int64_t kMinGroupTiles = 16;
 bool key_groups(int is_causal, int64_t head_dim, int64_t batch, int64_t q_heads, int64_t q_len, int64_t kv_len,
                 bool direct, int num_splits, int64_t ws_bytes) {

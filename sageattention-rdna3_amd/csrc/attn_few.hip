@@ -7,8 +7,8 @@
 // of K and V moved where 4 are read here), every query head of a group reads
 // K/V again, and 255 of a 256-row q-block's rows are padding.  At B8 Hq32
 // Hkv8 Sq1 Sk8192 D128 bf16 that took 74 us of prologue and 152 us of
-// attention, for K/V that a plain copy reads in 55 us; this kernel takes 55.4
-// us in all (4.85 TB/s of K and V).
+// attention, for K/V that a plain copy reads in 55 us; this kernel takes 55.8
+// us in all (4.81 TB/s of K and V).
 //
 // What bounds this kernel: the HBM reads of K and V (INT8 kind: with the
 // quantisation of K, ~7 VALU per element, close behind).  Mapping:

@@ -1,12 +1,13 @@
-// Compiled host layer of `sageattn` (the reference's sageattention/core.py:40-213
-// after its assertions): shapes and strides, the output / LSE / intermediate
-// allocations from the caller's torch allocator, and the launches through the
-// C ABI of libsage_mi355x.so, in one Python call.  The Python function keeps
-// the reference's assertions, its fp32 handling and the direct/INT8 dispatch
-// (with its environment overrides); everything after them runs here, because
-// for the short and cross-attention shapes the GPU work of a call (~12 us)
-// is smaller than what the same steps cost as Python (~10 us on top of the
-// launches).
+// Compiled host layer of `sageattn` (the reference's sageattention/core.py:40-213):
+// shapes and strides, the output / LSE / intermediate allocations from the
+// caller's torch allocator, and the launches through the C ABI of
+// libsage_mi355x.so, in one Python call, because for the short and
+// cross-attention shapes the GPU work of a call (~9 us) is smaller than what
+// the same steps cost as Python (~10 us on top of the launches).  A plain
+// fp16/bf16 call is checked and dispatched here too (sageattn_plain); any other
+// goes through the Python function, which holds the reference's assertions
+// with their messages, its fp32 handling and the direct/INT8 dispatch with its
+// environment overrides, and enters at sageattn_fwd.
 //
 // The module calls no HIP API itself: every launch goes through the C ABI on
 // the stream handle the caller passes (the current stream of the tensors'
@@ -116,7 +117,10 @@ constexpr int64_t kVRowsMaxQueriesCausal = 8192;
 // and quantises K again).  Whole call on MI355X, general / few in us, D64 fp16,
 // D128 bf16, H the (kv) heads of all batches; the lines below were drawn over
 // 4700 shapes of 4 to 1024 kv heads, 1 to 8 query heads each, 1 to 256 queries
-// and 32 to 16384 keys.
+// and 32 to 16384 keys.  One pass over K and V pays most where the general path
+// makes several: INT8 B8 Hq32 Hkv8 Sq1 Sk8192 D128 226 / 56, Hq64 Hkv8 Sq1
+// Sk8192 D64 33 / 25, H8 Sq256 Sk8192 D128 42 / 36.  More row tiles than these
+// lose: 16 (Sq512) 46 / 53; direct 4 of 128-row heads (H16 Sk2048 D128) 20 / 22.
 constexpr int64_t kFewMaxTiles = 8;
 constexpr int64_t kFewMaxTilesDirect = 3;   // direct path, heads of more than kFewShortHead rows
 constexpr int64_t kFewShortHead = 64;

@@ -87,7 +87,7 @@ def sageattn(
     q: [B,Hq,Sq,D] (HND) or [B,Sq,Hq,D] (NHD); k, v with Hkv heads (Hq % Hkv == 0).
     Returns o with q's shape, layout and dtype (and, when ``return_lse``, the
     rows' log-sum-exp [B,Hq,Sq] fp32: ln sum_j exp(sm_scale * q_i.k_j) after
-    quantisation, -inf for a row with no key; the reference returns zeros).
+    quantisation, -inf for a row with no key, NaN for a NaN row; the reference returns zeros).
     ``bm_sel`` (the reference's experimental direct-kernel tile override) is
     accepted and ignored; other unknown kwargs are ignored too.
     """
@@ -142,10 +142,11 @@ def sageattn(
 
     # the rest of the call (shapes, allocations, the launches of the direct or the INT8 path) in one
     # compiled call over the C ABI (csrc/host_ops.cpp): direct = one launch that reads V in place (the output of
-    # V transform + fp16_attn_t / bf16_attn_t, core.py:141-164, bit for bit); INT8 = [K mean] + K quantisation and
-    # V transform in one launch + the attention kernel that quantises Q itself (the q_int8 and q_scale of
-    # quant_qk_int8, so the same output); few queries = one launch for either.  return_lse: the reference returns a zero placeholder (core.py:203-211); both kernels
-    # write the real log-sum-exp of each row (natural log of the scaled scores; -inf without keys).
+    # V transform + fp16_attn_t / bf16_attn_t, core.py:141-164, bit for bit; long bf16 launches make the V transform);
+    # INT8 = [K mean] + K quantisation and V transform in one launch + the attention kernel that quantises Q itself
+    # (the q_int8 and q_scale of quant_qk_int8, so the same output); few queries = one launch for either.  return_lse:
+    # the reference returns a zero placeholder (core.py:203-211); the kernels write the real log-sum-exp of each row
+    # (natural log of the scaled scores; -inf without keys, NaN where the scores are NaN).
     with ops._on_device(q.device):
         res = _host().sageattn_fwd(q, k, v, layout_code, bool(is_causal), float(sm_scale), bool(return_lse),
                                    bool(kwargs.get("smooth_k", False)), direct,
