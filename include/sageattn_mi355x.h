@@ -181,8 +181,9 @@ int sage_attn_i8_fwd_lse(const int8_t* q_i8, const int8_t* k_i8, const void* val
  * rates 128-row q-blocks faster; R = 256 otherwise (one block per CU).
  * Non-causal 128-row blocks run two per CU, or one per CU in two key groups
  * where the launch has at most one item per CU and at least 16 key tiles an
- * item; causal ones one per CU in two key groups (more of them than CUs run as
- * a persistent grid, a heavy and a light q-block per block).  For a non-causal
+ * item; causal ones one per CU, in two key groups where a block has more than a
+ * few key tiles (more of them than CUs run as a persistent grid, a heavy and a
+ * light q-block per block).  For a non-causal
  * launch that leaves compute units idle
  * (fewer blocks than CUs, or a last round partly filled) the key range of
  * some or all blocks can be split into parts whose fp32 partial outputs and

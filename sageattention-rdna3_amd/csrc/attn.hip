@@ -78,14 +78,13 @@ namespace sage {
 //     per SIMD issues alone (a D = 64 direct step 1.9k cycles, against 3.0k for
 //     two tiles in g2).
 // The 128-row shapes run the D = 64 non-causal launches (direct and INT8) and
-// the causal launches with few q-blocks (small_blocks; all of those in g2, the
-// D = 64 ones as key_groups picks), w8 all others.  Same-box timings of w4
+// the causal launches with few q-blocks (small_blocks; key_groups picks w4 or
+// g2), w8 all others.  Same-box timings of w4
 // against w8 (identical outputs): D = 64 non-causal -7% to -27% (the direct
 // kernel at B1 H20 S1024: 21.3 -> 15.6 us; INT8 at B1 H10 S4096: 65.9 -> 56.2
 // us); causal launches of one or more full rounds +2% to +6% and D = 128
 // non-causal launches with key splits +3% to +4% (the doubled tile traffic),
-// so those stay on w8.  w4 / g2, whole sageattn, bf16, same box (causal w4 in a
-// build that has those kernels): INT8 causal B1 H8 S4096 D128 65.1 / 60.9 us,
+// so those stay on w8.  w4 / g2, whole sageattn, bf16, same box: INT8 causal B1 H8 S4096 D128 65.1 / 60.9 us,
 // H4 S8192 107.8 / 97.4, D64 H8 S6144 68.0 / 59.4; direct causal B1 H16 S2048
 // D128 40.7 / 37.6, H8 S1024 24.1 / 22.8, D64 H16 S2048 27.8 / 24.5; paired
 // causal: direct H32 S2048 D128 54.0 / 52.9, D64 33.7 / 30.8, INT8 H16 S4096
@@ -169,10 +168,14 @@ bool small_blocks(int64_t head_dim, int is_causal, int64_t batch, int64_t q_head
          w8::causal_blocks_cost<128, w8::kQkBf16>(batch * q_heads, q_len, kv_len);
 }
 
-// Whether a launch of 128-row q-blocks runs in g2 instead of w4: every causal
-// one (their blocks are alone on a CU in either shape), and a non-causal one
-// whose items (q-blocks, or key pieces of split ones) fit one per CU and have
-// at least this many key tiles.  With more items than CUs w4 hosts two blocks
+// Whether a launch of 128-row q-blocks runs in g2 instead of w4: a causal one
+// (their blocks are alone on a CU in either shape) whose heaviest q-block has
+// more key tiles than kMaxLoneTiles*, and a non-causal one whose items (q-blocks,
+// or key pieces of split ones) fit one per CU and have at least kMinGroupTiles.
+// Causal, whole call, w4 / g2, MI355X: direct fp16 B1 H8 S64 D64 5.8 / 6.9 us,
+// D128 7.5 / 8.8; S128 D128 9.6 / 10.3; S320 D64 8.4 / 8.8, D128 11.0 / 11.5; S384
+// even, S1024 D64 +7% in w4; INT8 fp16 S64 -15%, S320 D128 19.5 / 22.4, S512 -3% to
+// -11%, S640 -4% to +1%, S1280 D64 +6%.  Non-causal: with more items than CUs w4 hosts two blocks
 // a CU, which share no barrier (B1 H10 S4096 D64, 512 items: w4 60 us, g2 65);
 // with few tiles the merge and the doubled prologue outweigh the halved steps.
 // Whole call, w4 / g2, B1 H20 Sq1024 D64 (160 items; 80 to 240 items alike):
@@ -181,10 +184,15 @@ bool small_blocks(int64_t head_dim, int is_causal, int64_t batch, int64_t q_head
 // INT8 fp16 8 17.3 / 17.4, 16 22.1 / 21.2, 48 41.3 / 36.2.  Even at 12; from 16
 // on g2 gains in every kind.  Per piece of split items the same: H10, 2 or 3
 // pieces of 10 tiles 17.4 / 18.3, 3 of 16 29.3 / 28.9 (INT8).
+constexpr int64_t kMaxLoneTilesDirect = 5;
+constexpr int64_t kMaxLoneTilesI8 = 8;
 constexpr int64_t kMinGroupTiles = 16;
 bool key_groups(int is_causal, int64_t head_dim, int64_t batch, int64_t q_heads, int64_t q_len, int64_t kv_len,
                 bool direct, int num_splits, int64_t ws_bytes) {
-  if (is_causal != 0) return true;
+  if (is_causal != 0) {
+    const int64_t tiles = cdiv(std::min(cdiv(q_len, w4::kBM) * w4::kBM, kv_len), w4::kBN);
+    return tiles > (direct ? kMaxLoneTilesDirect : kMaxLoneTilesI8);
+  }
   const int64_t qblocks = batch * q_heads * cdiv(q_len, w4::kBM);
   if (qblocks <= 0 || qblocks > device_cus()) return false;
   const w4::SplitPlan sp = w4::plan_splits(!direct, qblocks, kv_len, head_dim, false, num_splits, ws_bytes);

@@ -2,7 +2,7 @@
 LDS) and the item decode's divisions, at the sizes where they can go wrong, through ``sageattn`` against the oracle.
 
 Non-causal launches run the shape from 16 key tiles on when their q-blocks fit one per compute unit; causal ones with
-few 256-row q-blocks at any length.  The cases: odd and even tile counts (an odd one leaves the second group a dead
+few 256-row q-blocks from 6 key tiles on (INT8 from 9), and the 4-wave 128-row shape below.  The cases: odd and even tile counts (an odd one leaves the second group a dead
 tile), a last tile of one key and of 64, one tile in all (the second group has none), rows past the last key and
 keys past the last row, one query, ragged query blocks, grouped heads, batch and head counts that are no power of two,
 D = 128 fp16/bf16 tiles (two ring stages a group), a forced key split, and persistent grids that pair q-blocks.
@@ -50,4 +50,30 @@ CASES = [
 @pytest.mark.parametrize("cfg,force_i8,splits", CASES, ids=[c[0].name for c in CASES])
 def test_key_groups_against_oracle(cfg, force_i8, splits, monkeypatch):
     monkeypatch.setenv("SAGEATTN_KV_SPLITS", str(splits))
+    check(cfg, force_i8, monkeypatch)
+
+
+# causal launches around the line between the 128-row shapes: one to five key tiles (INT8: to eight) run in 4-wave
+# blocks, longer ones in two key groups; the heaviest block's tiles count (few queries or few keys)
+SHORT = [
+    (case(0, 1, 2, 2, 1, 1, 64, "fp16", True), False),
+    (case(1, 2, 3, 1, 64, 64, 128, "bf16", True), False),
+    (case(2, 1, 5, 5, 100, 100, 64, "bf16", True), True),
+    (case(3, 3, 4, 2, 128, 128, 128, "fp16", True), False),
+    (case(4, 1, 3, 3, 129, 129, 128, "bf16", True), True),
+    (case(5, 1, 7, 7, 320, 320, 64, "fp16", True), False),
+    (case(6, 1, 4, 2, 321, 321, 128, "fp16", True), False),
+    (case(7, 1, 3, 3, 400, 2000, 64, "bf16", True), False),
+    (case(8, 1, 3, 3, 900, 330, 128, "bf16", True), False),
+    (case(9, 2, 3, 3, 900, 300, 64, "fp16", True, True), True),
+    (case(10, 1, 3, 3, 512, 512, 128, "bf16", True, True), True),
+    (case(11, 1, 6, 3, 513, 513, 64, "fp16", True), True),
+    (case(12, 1, 60, 60, 300, 300, 128, "bf16", True), False),
+    (case(13, 2, 64, 64, 300, 300, 64, "fp16", True), False),
+]
+
+
+@pytest.mark.parametrize("cfg,force_i8", SHORT, ids=[c[0].name for c in SHORT])
+def test_short_causal_against_oracle(cfg, force_i8, monkeypatch):
+    monkeypatch.delenv("SAGEATTN_KV_SPLITS", raising=False)
     check(cfg, force_i8, monkeypatch)

@@ -94,9 +94,9 @@ def test_few_queries_masked_keys_int8(D, monkeypatch):
 
 
 # block shapes of the general kernel: 128-row blocks in two key groups (17 key tiles), 128-row blocks (8), 256-row blocks,
-# causal 128-row blocks in two key groups
+# causal 128-row blocks in two key groups, causal 128-row blocks of few key tiles
 SHAPES = [(3, 300, 1088, 64, False), (5, 600, 512, 64, False), (3, 300, 700, 128, False), (3, 500, 500, 64, True),
-          (3, 500, 500, 128, True)]
+          (3, 500, 500, 128, True), (3, 300, 300, 64, True), (3, 300, 300, 128, True)]
 
 
 @pytest.mark.parametrize("low", [False, True])
@@ -132,7 +132,7 @@ def test_masked_keys_int8(H, Sq, Sk, D, masked, monkeypatch):
 NAN_CASES = [(4, 2, 3, 4096, 64, False, None), (4, 2, 3, 4096, 128, False, None), (4, 2, 3, 90, 128, False, None),
              (4, 2, 3, 90, 64, False, None), (4, 2, 300, 1088, 64, False, 1), (4, 2, 300, 1088, 64, False, 3),
              (4, 2, 300, 700, 128, False, 1), (4, 2, 300, 700, 128, False, 3), (4, 2, 300, 300, 128, True, None),
-             (4, 2, 300, 300, 64, True, None)]
+             (4, 2, 300, 300, 64, True, None), (4, 2, 600, 600, 128, True, None), (4, 2, 600, 600, 64, True, None)]
 NAN_IDS = [f"H{c[0]}q{c[2]}kv{c[3]}D{c[4]}{'_c' if c[5] else ''}_s{c[6]}" for c in NAN_CASES]
 
 
